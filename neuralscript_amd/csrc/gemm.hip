@@ -7,29 +7,35 @@
 // (CUDA counterparts ns_gemm_kernel / ns_grad_a_kernel / ns_grad_w_kernel,
 // /root/reference/src/codegen/cuda_backend.cpp:58-79, 446-467.)
 //
-// Design (wave64, MFMA 32x32x2 fp32, true fp32 products and sums):
-//  * 256-thread workgroup = 4 waves in a 2x2 grid; workgroup tile 128x128,
-//    wave tile 64x64 = 2x2 MFMA blocks of 32x32 (64 accumulators per lane).
-//  * K advances in 16-wide slabs staged in LDS, double buffered: the next
-//    slab's global loads are in flight while the current slab feeds the
-//    MFMAs; one barrier per slab.
-//  * Each operand keeps its global memory order in LDS (no transposing
-//    stores): k-contiguous operands are read back as float4 along k,
-//    row-contiguous operands as four scalars.  Within a 16-slab, lane half h
-//    of MFMA step q of group g consumes k = 8g + 4h + q for BOTH operands, a
-//    fixed bijection, so the contraction is unchanged.
-//  * Workgroup ids are remapped so each XCD (ids are dealt round-robin over
-//    the 8 XCDs) owns a contiguous run of tiles, grouped 8 tile-rows at a
-//    time for L2 reuse of the B panel.
-//  * The activation is applied to the accumulators before the single store.
+// Design (wave64).  Two kernels, one set of operand modes and epilogues:
+//  * gemm_bf3_kernel (16-byte aligned operands): fp32 products as six bf16
+//    MFMAs over three-piece operands (split3.h).  Operands are read as fp32,
+//    split in registers on their way to LDS, and each K slab of 16 is held
+//    there as [piece][k / 8][row] of 16-byte chunks, which is the MFMA operand
+//    order for either memory order of the operand (8 consecutive k of one row
+//    per lane), read back as conflict-free float4s.
+//  * gemm_f32_kernel (any alignment): fp32 MFMA 32x32x2, 128x128 tiles.
+//  * Both: K advances in 16-wide slabs staged in LDS, double buffered, one
+//    barrier per slab, global loads in flight under the MFMAs; workgroup ids
+//    are remapped so each XCD (ids are dealt round-robin over the 8 XCDs)
+//    owns a contiguous run of tiles, grouped 8 tile-rows at a time for L2
+//    reuse of the B panel; the epilogue works on the accumulators before the
+//    single store.
+//
+// The fp32 kernel keeps each operand's global memory order in LDS (no
+// transposing stores): k-contiguous operands are read back as float4 along k,
+// row-contiguous operands as four scalars.  Within a 16-slab, lane half h of
+// MFMA step q of group g consumes k = 8g + 4h + q for BOTH operands, a fixed
+// bijection, so the contraction is unchanged.
+#include <type_traits>
+
 #include "common.h"
 #include "kernels.h"
+#include "split3.h"
 
 namespace nship {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-constexpr int BM = 128, BN = 128, BK = 16;  // one 2x2-wave tile; the M side doubles with 4x2 waves
+constexpr int BM = 128, BN = 128, BK = 16;  // the fp32 kernel's tile (2x2 waves of 64x64)
 constexpr int KPAD = 4;    // pitch of k-contiguous rows: 20 floats
 constexpr int RPAD = 4;    // pitch of row-contiguous k rows: ROWS + 4 floats
 constexpr int NT = 256;
@@ -184,30 +190,30 @@ __device__ __forceinline__ void tile_of(int b, int tiles_m, int tiles_n, int& tm
   tn = in / gsize;
 }
 
-// Plain epilogue C = acc * act'(aux) for one wave's 64x64 block (aux with
-// C's row and column indices, pitch ldaux): the four 32x32 blocks' aux
+// Plain epilogue C = acc * act'(aux) for one wave's TM x TN blocks of 32x32
+// from (mw, nw) (aux with C's row and column indices, pitch ldaux): the aux
 // values are loaded one block ahead of that block's stores (the loads of
 // block b + 1 are in flight while block b is stored).  Its own loop nest, so
 // that the main epilogue's loops stay fully unrolled and the accumulators in
 // registers.
-template <int CODE>
-__device__ __forceinline__ void store_act_grad(const floatx16 (&acc)[2][2], const GemmArgs& g, float* __restrict__ C,
-                                               int m0, int n0, int wm, int wn, int l32, int kh, int m_end) {
+template <int CODE, int TM, int TN>
+__device__ __forceinline__ void store_act_grad(const floatx16 (&acc)[TM][TN], const GemmArgs& g, float* __restrict__ C,
+                                               int mw, int nw, int l32, int kh, int m_end) {
   if (g.mask_in) {
     // relu' from the sign bits: one 16-bit load per lane and 32x32 block,
     // bit v for the lane's accumulator v (the layout the forward wrote)
-    unsigned bits[4];
+    unsigned bits[TM * TN];
 #pragma unroll
-    for (int blk = 0; blk < 4; blk++) {
-      const int col = n0 + wn * 64 + (blk & 1) * 32 + l32;
-      const int rb = m0 + wm * 64 + (blk >> 1) * 32;
+    for (int blk = 0; blk < TM * TN; blk++) {
+      const int col = nw + (blk % TN) * 32 + l32;
+      const int rb = mw + (blk / TN) * 32;
       bits[blk] = col < g.N && rb < m_end ? g.mask_in[(int64_t)(2 * (rb / 32) + kh) * g.ldmask + col] : 0u;
     }
 #pragma unroll
-    for (int blk = 0; blk < 4; blk++) {
-      const int r = blk >> 1, c = blk & 1;
-      const int col = n0 + wn * 64 + c * 32 + l32;
-      const int row0 = m0 + wm * 64 + r * 32 + 4 * kh;
+    for (int blk = 0; blk < TM * TN; blk++) {
+      const int r = blk / TN, c = blk % TN;
+      const int col = nw + c * 32 + l32;
+      const int row0 = mw + r * 32 + 4 * kh;
       const bool cin = col < g.N;
       float* cp = C + (int64_t)row0 * g.ldc + col;
 #pragma unroll
@@ -220,8 +226,8 @@ __device__ __forceinline__ void store_act_grad(const floatx16 (&acc)[2][2], cons
   }
   float au[2][16];
   auto load = [&](int blk, float(&dst)[16]) {
-    const int col = n0 + wn * 64 + (blk & 1) * 32 + l32;
-    const int row0 = m0 + wm * 64 + (blk >> 1) * 32 + 4 * kh;
+    const int col = nw + (blk % TN) * 32 + l32;
+    const int row0 = mw + (blk / TN) * 32 + 4 * kh;
     const bool cin = col < g.N;
     const float* ap = g.aux + (int64_t)row0 * g.ldaux + col;
 #pragma unroll
@@ -232,11 +238,11 @@ __device__ __forceinline__ void store_act_grad(const floatx16 (&acc)[2][2], cons
   };
   load(0, au[0]);
 #pragma unroll
-  for (int blk = 0; blk < 4; blk++) {
-    if (blk + 1 < 4) load(blk + 1, au[(blk + 1) & 1]);
-    const int r = blk >> 1, c = blk & 1;
-    const int col = n0 + wn * 64 + c * 32 + l32;
-    const int row0 = m0 + wm * 64 + r * 32 + 4 * kh;
+  for (int blk = 0; blk < TM * TN; blk++) {
+    if (blk + 1 < TM * TN) load(blk + 1, au[(blk + 1) & 1]);
+    const int r = blk / TN, c = blk % TN;
+    const int col = nw + c * 32 + l32;
+    const int row0 = mw + r * 32 + 4 * kh;
     const bool cin = col < g.N;
     float* cp = C + (int64_t)row0 * g.ldc + col;
 #pragma unroll
@@ -250,14 +256,15 @@ __device__ __forceinline__ void store_act_grad(const floatx16 (&acc)[2][2], cons
 // Sign bits of the pre-activation for a relu gradient later (the layout of
 // GemmArgs::mask_out): each lane's 16 rows of a 32x32 block in one 16-bit
 // value.  Its own loop nest, as store_act_grad.
-__device__ __forceinline__ void store_relu_bits(const floatx16 (&acc)[2][2], const GemmArgs& g, int m0, int n0, int wm,
-                                                int wn, int l32, int kh, int m_end) {
+template <int TM, int TN>
+__device__ __forceinline__ void store_relu_bits(const floatx16 (&acc)[TM][TN], const GemmArgs& g, int mw, int nw,
+                                                int l32, int kh, int m_end) {
 #pragma unroll
-  for (int r = 0; r < 2; r++)
+  for (int r = 0; r < TM; r++)
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
-      const int col = n0 + wn * 64 + c * 32 + l32;
-      const int rb = m0 + wm * 64 + r * 32;
+    for (int c = 0; c < TN; c++) {
+      const int col = nw + c * 32 + l32;
+      const int rb = mw + r * 32;
       unsigned bits = 0u;
 #pragma unroll
       for (int v = 0; v < 16; v++) bits |= (acc[r][c][v] > 0.f ? 1u : 0u) << v;
@@ -265,53 +272,43 @@ __device__ __forceinline__ void store_relu_bits(const floatx16 (&acc)[2][2], con
     }
 }
 
-// opA(A)[m,k]: TA ? A[k*lda+m] : A[m*lda+k]   (KC for A <=> !TA)
-// opB(B)[k,n]: TB ? B[n*ldb+k] : B[k*ldb+n]   (KC for B <=>  TB)
-// PLAIN: no row scatter, no row scale; epilogue kEpiAct (with the
-// pre-activation / activation pair when C2 is set), kEpiActGrad or kEpiAccum.
-// WMW = 2 / WNW = 2: 4x2 / 2x4 waves (512 threads), workgroup tile
-// 256 x 128 / 128 x 256: a quarter fewer operand loads and LDS stores per FLOP.
-template <bool TA, bool TB, bool VEC, bool PLAIN, int WMW, int WNW>
-__global__ __launch_bounds__(NT * WMW * WNW, VEC ? 4 / (WMW * WNW) : 1) void gemm_f32_kernel(GemmArgs g) {
-  constexpr int BMT = BM * WMW, BNT = BN * WNW, NTT = NT * WMW * WNW;
-  const int M = g.M, N = g.N, K = g.K;
-  const int64_t lda = g.lda, ldb = g.ldb, ldc = g.ldc;
-  const int tiles_m = g.tiles_m, tiles_n = g.tiles_n;
-  const float* __restrict__ A = g.A + (int64_t)blockIdx.y * g.sA;
-  const float* __restrict__ B = g.B + (int64_t)blockIdx.y * g.sB;
-  float* __restrict__ C = g.C + (int64_t)blockIdx.y * g.sC;
-  int m_end = M;
+// What one workgroup computes: C[m0.., n0..] over k in [kbeg, kend).
+struct Job {
+  const float* A;
+  const float* B;
+  float* C;
+  int kbeg, kend, m0, n0, m_end;
+};
+
+// The job of this workgroup under g's mode (batch, K-grouped, K-chunked,
+// split K, grouped) for BMT x BNT tiles; false: nothing to do (uniform).
+template <int BMT, int BNT>
+__device__ __forceinline__ bool tile_job(const GemmArgs& g, Job& j) {
+  j.A = g.A + (int64_t)blockIdx.y * g.sA;
+  j.B = g.B + (int64_t)blockIdx.y * g.sB;
+  j.C = g.C + (int64_t)blockIdx.y * g.sC;
+  j.m_end = g.M;
   // K-grouped: group blockIdx.y contracts over k in [kseg[y], kseg[y+1]).
-  int kbeg = 0, kend = K;
+  j.kbeg = 0;
+  j.kend = g.K;
   if (g.kseg) {
-    kbeg = g.kseg[blockIdx.y];
-    kend = g.kseg[blockIdx.y + 1];
+    j.kbeg = g.kseg[blockIdx.y];
+    j.kend = g.kseg[blockIdx.y + 1];
   }
   if (g.kitems) {
-    if ((int)blockIdx.y >= *g.nkitems) return;
+    if ((int)blockIdx.y >= *g.nkitems) return false;
     const int* it = g.kitems + 4 * blockIdx.y;
-    kbeg = it[1];
-    kend = it[2];
-    A = g.A;
-    B = g.B;
-    C = it[3] < 0 ? g.C + (int64_t)it[0] * g.sC : g.kpart + (int64_t)it[3] * g.sC;
+    j.kbeg = it[1];
+    j.kend = it[2];
+    j.A = g.A;
+    j.B = g.B;
+    j.C = it[3] < 0 ? g.C + (int64_t)it[0] * g.sC : g.kpart + (int64_t)it[3] * g.sC;
   }
   if (g.kchunk) {
-    kbeg = (int)blockIdx.z * g.kchunk;
-    kend = min(K, kbeg + g.kchunk);
-    C += (int64_t)blockIdx.z * g.sCk;
+    j.kbeg = (int)blockIdx.z * g.kchunk;
+    j.kend = min(g.K, j.kbeg + g.kchunk);
+    j.C += (int64_t)blockIdx.z * g.sCk;
   }
-  constexpr bool AKC = !TA, BKC = TB;
-  constexpr int ASZ = TileLayout<AKC, BMT>::kSize, BSZ = TileLayout<BKC, BNT>::kSize;
-  __shared__ __attribute__((aligned(16))) float smem[2 * (ASZ + BSZ)];
-  // buffer b: A tile at smem + b*(ASZ+BSZ), B tile right after it
-
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  const int wm = wave / (2 * WNW), wn = wave % (2 * WNW);
-  const int l32 = lane & 31, kh = lane >> 5;
-
-  int m0, n0;
   if (g.groups) {
     // Grouped: tile entry -> (group, m tile); rows [seg[e], seg[e+1]) of the
     // group, B advanced by e * sBg.  Entries run XCD-contiguously with all
@@ -319,36 +316,58 @@ __global__ __launch_bounds__(NT * WMW * WNW, VEC ? 4 / (WMW * WNW) : 1) void gem
     // The grid is an upper bound: the workgroups past the device-side tile
     // count exit (uniformly), and the rest are spread over the 8 XCDs by
     // that count, not by the grid size, so each XCD gets an equal share.
-    const int T = *g.ntiles * tiles_n;
-    if ((int)blockIdx.x >= T) return;
+    const int T = *g.ntiles * g.tiles_n;
+    if ((int)blockIdx.x >= T) return false;
     const int L = xcd_linear(blockIdx.x, T);
-    const int entry = L / tiles_n;
+    const int entry = L / g.tiles_n;
     const int e = g.tiles[2 * entry], mt = g.tiles[2 * entry + 1];
-    m0 = g.seg[e] + mt * BMT;
-    m_end = g.seg[e + 1];
-    n0 = (L % tiles_n) * BNT;
-    B += (int64_t)e * g.sBg;
+    j.m0 = g.seg[e] + mt * BMT;
+    j.m_end = g.seg[e + 1];
+    j.n0 = (L % g.tiles_n) * BNT;
+    j.B += (int64_t)e * g.sBg;
   } else {
     int tm, tn;
-    tile_of(blockIdx.x, tiles_m, tiles_n, tm, tn);
-    m0 = tm * BMT;
-    n0 = tn * BNT;
+    tile_of(blockIdx.x, g.tiles_m, g.tiles_n, tm, tn);
+    j.m0 = tm * BMT;
+    j.n0 = tn * BNT;
   }
+  return true;
+}
 
-  floatx16 acc[2][2];
+template <int TM, int TN>
+__device__ __forceinline__ void zero_acc(floatx16 (&acc)[TM][TN]) {
 #pragma unroll
-  for (int r = 0; r < 2; r++)
+  for (int r = 0; r < TM; r++)
 #pragma unroll
-    for (int c = 0; c < 2; c++)
+    for (int c = 0; c < TN; c++)
 #pragma unroll
       for (int v = 0; v < 16; v++) acc[r][c][v] = 0.f;
+}
 
+// Floats of LDS the fp32 loop needs for a BMT x BNT tile.
+template <bool TA, bool TB, int BMT, int BNT>
+constexpr int f32_lds_floats() {
+  return 2 * (TileLayout<!TA, BMT>::kSize + TileLayout<TB, BNT>::kSize);
+}
+
+// fp32-MFMA K loop of one tile, WM x WN waves of TM x TN 32x32 blocks.
+template <bool TA, bool TB, bool VEC, int WM, int WN, int TM, int TN>
+__device__ __forceinline__ void mainloop_f32(const GemmArgs& g, const Job& j, float* __restrict__ smem,
+                                             floatx16 (&acc)[TM][TN]) {
+  constexpr int BMT = 32 * WM * TM, BNT = 32 * WN * TN, NTT = 64 * WM * WN;
+  constexpr bool AKC = !TA, BKC = TB;
+  constexpr int ASZ = TileLayout<AKC, BMT>::kSize, BSZ = TileLayout<BKC, BNT>::kSize;
+  // buffer b: A tile at smem + b*(ASZ+BSZ), B tile right after it
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int wm = wave / WN, wn = wave % WN, l32 = lane & 31, kh = lane >> 5;
+  const int64_t lda = g.lda, ldb = g.ldb;
+  const int kbeg = j.kbeg, kend = j.kend;
+  zero_acc(acc);
   Stage<AKC, VEC, BMT, NTT> sa;
   Stage<BKC, VEC, BNT, NTT> sb;
   const int nk = (kend - kbeg + BK - 1) / BK;
-  // (the 256-row tiles never gather rows)
-  sa.init(A, lda, m0, m_end, t, WMW == 2 ? nullptr : g.a_rows);
-  sb.init(B, ldb, n0, N, t);
+  sa.init(j.A, lda, j.m0, j.m_end, t, g.a_rows);
+  sb.init(j.B, ldb, j.n0, g.N, t);
   sa.kblk_ = g.kblk;
   sa.sk_ = g.sAk;
   sb.kblk_ = g.kblk;
@@ -359,7 +378,7 @@ __global__ __launch_bounds__(NT * WMW * WNW, VEC ? 4 / (WMW * WNW) : 1) void gem
   sb.store(smem + ASZ, t);
   __syncthreads();
   // every row and K slab of the tile in range: loads without checks
-  const bool full = m0 + BMT <= m_end && n0 + BNT <= N && (kend - kbeg) % BK == 0;
+  const bool full = j.m0 + BMT <= j.m_end && j.n0 + BNT <= g.N && (kend - kbeg) % BK == 0;
 
   for (int kt = 0; kt < nk; kt++) {
     const int cur = kt & 1;
@@ -376,23 +395,20 @@ __global__ __launch_bounds__(NT * WMW * WNW, VEC ? 4 / (WMW * WNW) : 1) void gem
     const float* as = smem + cur * (ASZ + BSZ);
     const float* bs = as + ASZ;
     __builtin_amdgcn_s_setprio(1);
-    // the scheduler's MFMA / LDS-read interleaving for GEMM loops: +0.5-0.9%
-    // on the 256-row tiles, slower on the others (c5's 128x128 products -21%)
-    if constexpr (WMW == 2) __builtin_amdgcn_iglp_opt(1);
 #pragma unroll
-    for (int g = 0; g < 2; g++) {
-      const int kb = 8 * g + 4 * kh;
-      float fa[2][4], fb[2][4];
+    for (int g2 = 0; g2 < 2; g2++) {
+      const int kb = 8 * g2 + 4 * kh;
+      float fa[TM][4], fb[TN][4];
 #pragma unroll
-      for (int r = 0; r < 2; r++) read_frag<AKC, BMT>(as, wm * 64 + r * 32 + l32, kb, fa[r]);
+      for (int r = 0; r < TM; r++) read_frag<AKC, BMT>(as, (wm * TM + r) * 32 + l32, kb, fa[r]);
 #pragma unroll
-      for (int c = 0; c < 2; c++) read_frag<BKC, BNT>(bs, wn * 64 + c * 32 + l32, kb, fb[c]);
+      for (int c = 0; c < TN; c++) read_frag<BKC, BNT>(bs, (wn * TN + c) * 32 + l32, kb, fb[c]);
 #pragma unroll
       for (int q = 0; q < 4; q++)
 #pragma unroll
-        for (int r = 0; r < 2; r++)
+        for (int r = 0; r < TM; r++)
 #pragma unroll
-          for (int c = 0; c < 2; c++)
+          for (int c = 0; c < TN; c++)
             acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[r][q], fb[c][q], acc[r][c], 0, 0, 0);
     }
     __builtin_amdgcn_s_setprio(0);
@@ -403,24 +419,36 @@ __global__ __launch_bounds__(NT * WMW * WNW, VEC ? 4 / (WMW * WNW) : 1) void gem
     }
     __syncthreads();
   }
+}
 
+// Epilogue of one wave's TM x TN 32x32 blocks, the first at (mw, nw).
+// PLAIN: no row scatter, no row scale; epilogue kEpiAct (with the
+// pre-activation / activation pair when C2 is set), kEpiActGrad or kEpiAccum.
+// ACTS: bit c set = activation c may be asked for (each costs a copy of the
+// stores of every accumulator).
+constexpr unsigned kAllActs = 0xff;
+template <bool PLAIN, unsigned ACTS, int TM, int TN>
+__device__ __forceinline__ void store_tile(const floatx16 (&acc)[TM][TN], const GemmArgs& g, float* __restrict__ C,
+                                           int mw, int nw, int l32, int kh, int m_end) {
+  const int N = g.N;
+  const int64_t ldc = g.ldc;
   // Accumulator v of lane (l32, kh) in a 32x32 block sits at
   // row 8*(v/4) + 4*kh + v%4, column l32.
   if constexpr (PLAIN) {
     if (g.mode == kEpiActGrad) {
       // C = acc * relu'(aux): the only activation gradient the plain path
       // takes (plain_act_grad)
-      store_act_grad<kActRelu>(acc, g, C, m0, n0, wm, wn, l32, kh, m_end);
+      store_act_grad<kActRelu>(acc, g, C, mw, nw, l32, kh, m_end);
       return;
     }
-    if (g.mask_out) store_relu_bits(acc, g, m0, n0, wm, wn, l32, kh, m_end);
+    if (g.mask_out) store_relu_bits(acc, g, mw, nw, l32, kh, m_end);
     // plain stores, the activation resolved once per 32x32 block
 #pragma unroll
-    for (int r = 0; r < 2; r++)
+    for (int r = 0; r < TM; r++)
 #pragma unroll
-      for (int c = 0; c < 2; c++) {
-        const int col = n0 + wn * 64 + c * 32 + l32;
-        const int row0 = m0 + wm * 64 + r * 32 + 4 * kh;
+      for (int c = 0; c < TN; c++) {
+        const int col = nw + c * 32 + l32;
+        const int row0 = mw + r * 32 + 4 * kh;
         float* cp = C + (int64_t)row0 * ldc + col;
         const bool cin = col < N;
 #define NSH_STORE16(CODE)                                                          \
@@ -446,13 +474,13 @@ __global__ __launch_bounds__(NT * WMW * WNW, VEC ? 4 / (WMW * WNW) : 1) void gem
           cp = g.C2 + (int64_t)blockIdx.y * g.sC + (int64_t)row0 * ldc + col;
         }
         switch (g.act) {
-          case kActRelu: NSH_STORE16(kActRelu); break;
-          case kActLeaky: NSH_STORE16(kActLeaky); break;
-          case kActSigmoid: NSH_STORE16(kActSigmoid); break;
-          case kActTanh: NSH_STORE16(kActTanh); break;
-          case kActSilu: NSH_STORE16(kActSilu); break;
-          case kActGelu: NSH_STORE16(kActGelu); break;
-          case kActGeluMoe: NSH_STORE16(kActGeluMoe); break;
+          case kActRelu: if constexpr ((ACTS >> kActRelu) & 1) { NSH_STORE16(kActRelu); } break;
+          case kActLeaky: if constexpr ((ACTS >> kActLeaky) & 1) { NSH_STORE16(kActLeaky); } break;
+          case kActSigmoid: if constexpr ((ACTS >> kActSigmoid) & 1) { NSH_STORE16(kActSigmoid); } break;
+          case kActTanh: if constexpr ((ACTS >> kActTanh) & 1) { NSH_STORE16(kActTanh); } break;
+          case kActSilu: if constexpr ((ACTS >> kActSilu) & 1) { NSH_STORE16(kActSilu); } break;
+          case kActGelu: if constexpr ((ACTS >> kActGelu) & 1) { NSH_STORE16(kActGelu); } break;
+          case kActGeluMoe: if constexpr ((ACTS >> kActGeluMoe) & 1) { NSH_STORE16(kActGeluMoe); } break;
           default: NSH_STORE16(kActId); break;
         }
 #undef NSH_STORE16
@@ -464,13 +492,13 @@ __global__ __launch_bounds__(NT * WMW * WNW, VEC ? 4 / (WMW * WNW) : 1) void gem
   // row and scale between the two column blocks: they are looked up once,
   // eight rows at a time with all eight loads in flight together.
 #pragma unroll
-  for (int r = 0; r < 2; r++)
+  for (int r = 0; r < TM; r++)
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-      const int rbase = m0 + wm * 64 + r * 32 + 16 * h + 4 * kh;
+      const int rbase = mw + r * 32 + 16 * h + 4 * kh;
       int crow[8];
       float rs[8];
-      // rows past m_end read row m_end - 1's entries (m0 < m_end) and are
+      // rows past m_end read row m_end - 1's entries (the tile has rows) and are
       // then marked -1: the loads carry no branch and issue together
 #pragma unroll
       for (int u = 0; u < 8; u++) crow[u] = min(rbase + 8 * (u >> 2) + (u & 3), m_end - 1);
@@ -484,8 +512,8 @@ __global__ __launch_bounds__(NT * WMW * WNW, VEC ? 4 / (WMW * WNW) : 1) void gem
       for (int u = 0; u < 8; u++)
         if (rbase + 8 * (u >> 2) + (u & 3) >= m_end) crow[u] = -1;
 #pragma unroll
-      for (int c = 0; c < 2; c++) {
-        const int col = n0 + wn * 64 + c * 32 + l32;
+      for (int c = 0; c < TN; c++) {
+        const int col = nw + c * 32 + l32;
         if (col >= N) continue;
 #pragma unroll
         for (int u = 0; u < 8; u++) {
@@ -494,12 +522,278 @@ __global__ __launch_bounds__(NT * WMW * WNW, VEC ? 4 / (WMW * WNW) : 1) void gem
           float* dst = C + (int64_t)crow[u] * ldc + col;
           const float x = acc[r][c][8 * h + u];
           const float a = g.row_scale ? x * rs[u] : x;
-          if (g.mode == kEpiAct) *dst = act_apply(a, g.act);
-          else if (g.mode == kEpiActGrad) *dst = a * act_deriv(g.aux[(int64_t)row * g.ldaux + col], g.act);
-          else *dst = *dst + a;
+          if (g.mode == kEpiAccum) {
+            *dst = *dst + a;
+          } else if constexpr (ACTS == 1u) {
+            *dst = a;
+          } else {
+            if (g.mode == kEpiAct) *dst = act_apply(a, g.act);
+            else *dst = a * act_deriv(g.aux[(int64_t)row * g.ldaux + col], g.act);
+          }
         }
       }
     }
+}
+
+// opA(A)[m,k]: TA ? A[k*lda+m] : A[m*lda+k]   (KC for A <=> !TA)
+// opB(B)[k,n]: TB ? B[n*ldb+k] : B[k*ldb+n]   (KC for B <=>  TB)
+// The fp32 kernel: 256 threads = 2x2 waves of 64x64.  It takes what the split
+// kernel does not (bf3_takes): operands that cannot be read as float4, and
+// products too small to be worth the split.
+template <bool TA, bool TB, bool VEC, bool PLAIN>
+__global__ __launch_bounds__(NT, VEC ? 4 : 1) void gemm_f32_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) float smem[f32_lds_floats<TA, TB, BM, BN>()];
+  Job j;
+  if (!tile_job<BM, BN>(g, j)) return;
+  floatx16 acc[2][2];
+  mainloop_f32<TA, TB, VEC, 2, 2, 2, 2>(g, j, smem, acc);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  store_tile<PLAIN, kAllActs>(acc, g, j.C, j.m0 + (wave >> 1) * 64, j.n0 + (wave & 1) * 64, lane & 31, lane >> 5, j.m_end);
+}
+
+// ---- three-piece bf16 kernel ---------------------------------------------------
+
+// Operands are scaled by 2^24 before they are split, and the accumulators by
+// 2^-48 after the K loop (all exact): the last piece then stays above bf16's
+// smallest subnormal for every fp32 operand down to 2^-134, so a gradient's
+// softmax tails do not take the fp32 path.  The scaled sums overflow where a
+// result exceeds 2^80; such tiles take the fp32 path too.
+constexpr float kSplitUp = 0x1p24f, kSplitDown = 0x1p-48f;
+
+// LDS layout of one operand's 16-wide K slab: [piece][k / 8][row] chunks of 8
+// bf16.  The two k-halves are 64 bytes further apart than ROWS chunks, so the
+// staging stores of a k-contiguous operand (8 lanes = 4 rows x 2 halves)
+// cover all banks.
+template <int ROWS>
+struct Bf3Layout {
+  static constexpr int kHalf = ROWS * 16 + 64;
+  static constexpr int kPiece = 2 * kHalf;
+  static constexpr int kBytes = 3 * kPiece;
+};
+
+// Global -> register -> LDS staging of one ROWS x 16 slab by NTH threads, W
+// consecutive k of one row at a time: two float4 of a k-contiguous operand,
+// or W loads a row pitch apart of a row-contiguous one, whose consecutive
+// rows lie in consecutive lanes.  The slabs are taken in order.  No load and
+// no step between slabs branches, so the K loop's body is one block in which
+// the split of one slab is scheduled among the MFMAs of another: CHK = true
+// (rows or a K slab past the end) reads from an address in range instead and
+// puts zeros in at the store.
+template <bool KC, int ROWS, int NTH>
+struct Bf3Stage {
+  static constexpr int W = ROWS * 2 >= NTH ? 8 : 4;
+  static constexpr int NC = BK / W;             // W-chunks of a slab
+  static constexpr int kN = ROWS * NC / NTH;    // chunks per thread
+  static_assert(kN >= 1 && kN * NTH == ROWS * NC, "the chunks divide evenly");
+  float v[kN][W];
+  const float* p[kN];  // chunk i of slab 0: its row (in range), or (KC false) the tile's first row
+  uint32_t ro[kN];     // KC false: byte offset of chunk i's row (in range) from there
+  unsigned rin;        // bit i set: the row of chunk i is in range
+  int64_t off, wrap;   // of the next slab; what the end of a K block adds
+  int k, inblk, kblk;  // next slab, its place in its K block, the block's length
+  int lim;             // k of the held slab below lim exist
+
+  __device__ __forceinline__ static void pos(int idx, int& r, int& kc) {
+    // (KC false: ROWS is a multiple of the wave, so kc is uniform and the
+    // loads' addresses are scalar but for the row offset)
+    if (KC) { r = idx / NC; kc = idx % NC; } else { kc = __builtin_amdgcn_readfirstlane(idx / ROWS); r = idx % ROWS; }
+  }
+  // rmap (optional, KC): row r of the operand is row rmap[r] of `base`.  kb > 0:
+  // K blocks of kb steps, sk floats apart.
+  __device__ __forceinline__ void init(const float* __restrict__ base, int64_t ld, int row0, int rows, int kbeg, int t,
+                                       const int* __restrict__ rmap, int kb, int64_t sk) {
+    rin = 0;
+#pragma unroll
+    for (int i = 0; i < kN; i++) {
+      int r, kc;
+      pos(t + NTH * i, r, kc);
+      const int gr = row0 + r;
+      const bool in = gr < rows;
+      rin |= in ? 1u << i : 0u;
+      if (KC) {
+        p[i] = base + (!in ? 0 : rmap ? (int64_t)rmap[gr] : (int64_t)gr) * ld;
+      } else {
+        p[i] = base + row0 + (int64_t)(kc * W) * ld;
+        ro[i] = (uint32_t)min(r, rows - 1 - row0) * 4u;
+      }
+    }
+    kblk = kb > 0 ? kb : INT32_MAX;
+    k = kbeg;
+    inblk = kb > 0 ? kbeg % kb : kbeg;
+    const int64_t unit = KC ? 1 : ld;
+    wrap = kb > 0 ? sk - kb * unit : 0;
+    off = (kb > 0 ? kbeg / kb * wrap : 0) + kbeg * unit;
+  }
+  // The next slab, then on by one; past the last one (k >= kend - BK) it stays
+  // (nothing reads the slab then loaded again).
+  template <bool CHK>
+  __device__ __forceinline__ void load(int64_t ld, int kend, int t) {
+    lim = kend - k;
+#pragma unroll
+    for (int i = 0; i < kN; i++) {
+      int r, kc;
+      pos(t + NTH * i, r, kc);
+      if (KC) {
+#pragma unroll
+        for (int u = 0; u < W; u += 4) {
+          // (whole float4: kend and k are multiples of 4)
+          const int ku = CHK ? min(kc * W + u, lim - 4) : kc * W + u;
+          const float4 x = *reinterpret_cast<const float4*>(p[i] + off + ku);
+          v[i][u] = x.x; v[i][u + 1] = x.y; v[i][u + 2] = x.z; v[i][u + 3] = x.w;
+        }
+      } else {
+        const float* q = p[i] + off;
+#pragma unroll
+        for (int u = 0; u < W; u++) {
+          if (CHK) q = p[i] + off + (int64_t)min(u, lim - 1 - kc * W) * ld;
+          v[i][u] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(q) + ro[i]);
+          if (!CHK) q += ld;
+        }
+      }
+    }
+    const bool more = k + BK < kend;
+    k += more ? BK : 0;
+    off += more ? (KC ? (int64_t)BK : BK * ld) : 0;
+    inblk += more ? BK : 0;
+    const bool next = inblk >= kblk;
+    off += next ? wrap : 0;
+    inblk = next ? 0 : inblk;
+  }
+  template <bool CHK>
+  __device__ __forceinline__ void store(char* __restrict__ lds, int t, bool& bad) {
+    using L = Bf3Layout<ROWS>;
+#pragma unroll
+    for (int i = 0; i < kN; i++) {
+      int r, kc;
+      pos(t + NTH * i, r, kc);
+      uint32_t w0[W / 2], w1[W / 2], w2[W / 2];
+#pragma unroll
+      for (int u = 0; u < W; u++) {
+        if (CHK) v[i][u] = ((rin >> i) & 1) && kc * W + u < lim ? v[i][u] : 0.f;
+        v[i][u] *= kSplitUp;
+      }
+      split_run<W>(v[i], w0, w1, w2, bad);
+      if constexpr (W == 8) {
+        char* d = lds + kc * L::kHalf + r * 16;
+        *reinterpret_cast<uintx4*>(d) = uintx4{w0[0], w0[1], w0[2], w0[3]};
+        *reinterpret_cast<uintx4*>(d + L::kPiece) = uintx4{w1[0], w1[1], w1[2], w1[3]};
+        *reinterpret_cast<uintx4*>(d + 2 * L::kPiece) = uintx4{w2[0], w2[1], w2[2], w2[3]};
+      } else {
+        char* d = lds + (kc >> 1) * L::kHalf + r * 16 + (kc & 1) * 8;
+        *reinterpret_cast<uintx2*>(d) = uintx2{w0[0], w0[1]};
+        *reinterpret_cast<uintx2*>(d + L::kPiece) = uintx2{w1[0], w1[1]};
+        *reinterpret_cast<uintx2*>(d + 2 * L::kPiece) = uintx2{w2[0], w2[1]};
+      }
+    }
+  }
+};
+
+// The activations that the split kernel's epilogues hold, by use: a dense
+// layer's (NN) all; transposed products (gradients) and the general epilogue
+// none; an expert layer's GELU.  bf3_takes sends the rest elsewhere.
+constexpr unsigned kActsNone = 1u << kActId;
+constexpr unsigned kActsMoe = 1u << kActId | 1u << kActGeluMoe;
+
+// WM x WN waves, each 2 x 2 blocks of 32x32.
+//
+// Two accumulators a block: `acc` takes the products of the leading pieces,
+// `lo` the other five, and they are added once at the end.  An MFMA aligns its
+// products to its accumulator and truncates below two guard bits, which
+// shrinks sums of mixed sign by about 2^-27 sqrt(K); in `lo`, 2^-8 the size,
+// both that and the roundings vanish, and `acc` is rounded once per 16 of K.
+// Error against float64, one accumulator -> two (fp32 MFMA): K = 4096 1.0e-6
+// -> 4.0e-7 (1.1e-6), K = 512 3.4e-7 -> 1.3e-7 (4.1e-7).
+//
+// Bound by the matrix cores and the power they draw: a register-only loop of
+// the same MFMAs runs at 1.8 PFLOP/s, 300 TFLOP/s of fp32 products; 8192 x
+// 4096 x 4096 runs at 216 (fp32 MFMA 127), 16384 x 512 x 8192 at 203 (126).
+// 64x64 per wave is what two accumulators leave room for at two waves per
+// SIMD; 128x64 per wave with one accumulator ran at 234, with the error above.
+// The slab after next is loaded right after its registers were split and
+// stored, so a load has a whole slab of MFMAs to arrive.
+template <bool TA, bool TB, bool PLAIN, unsigned ACTS, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf3_kernel(GemmArgs g) {
+  constexpr int TM = 2, TN = 2;
+  constexpr int BMT = 32 * WM * TM, BNT = 32 * WN * TN, NTT = 64 * WM * WN;
+  using LA = Bf3Layout<BMT>;
+  using LB = Bf3Layout<BNT>;
+  constexpr int kBuf = LA::kBytes + LB::kBytes;
+  constexpr int kF32 = 4 * f32_lds_floats<TA, TB, BMT, BNT>();
+  __shared__ __attribute__((aligned(16))) char smem[2 * kBuf > kF32 ? 2 * kBuf : kF32];
+  Job j;
+  if (!tile_job<BMT, BNT>(g, j)) return;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int wm = wave / WN, wn = wave % WN, l32 = lane & 31, kh = lane >> 5;
+  const int kbeg = j.kbeg, kend = j.kend, nk = (kend - kbeg + BK - 1) / BK;
+  const int64_t lda = g.lda, ldb = g.ldb;
+  floatx16 acc[TM][TN];
+  zero_acc(acc);
+  bool bad = false;
+  {
+    floatx16 lo[TM][TN];
+    zero_acc(lo);
+    auto kloop = [&](auto chk) {
+      constexpr bool CHK = decltype(chk)::value;
+      Bf3Stage<!TA, BMT, NTT> sa;
+      Bf3Stage<TB, BNT, NTT> sb;
+      sa.init(j.A, lda, j.m0, j.m_end, kbeg, t, g.a_rows, g.kblk, g.sAk);
+      sb.init(j.B, ldb, j.n0, g.N, kbeg, t, nullptr, g.kblk, g.sBk);
+      sa.template load<CHK>(lda, kend, t);
+      sb.template load<CHK>(ldb, kend, t);
+      sa.template store<CHK>(smem, t, bad);
+      sb.template store<CHK>(smem + LA::kBytes, t, bad);
+      sa.template load<CHK>(lda, kend, t);
+      sb.template load<CHK>(ldb, kend, t);
+      __syncthreads();
+      for (int kt = 0; kt < nk; kt++) {
+        const char* as = smem + (kt & 1) * kBuf + kh * LA::kHalf + (wm * TM * 32 + l32) * 16;
+        const char* bs = smem + (kt & 1) * kBuf + LA::kBytes + kh * LB::kHalf + (wn * TN * 32 + l32) * 16;
+        bf16x8 fb[TN][3];
+#pragma unroll
+        for (int c = 0; c < TN; c++)
+#pragma unroll
+          for (int p = 0; p < 3; p++) fb[c][p] = *reinterpret_cast<const bf16x8*>(bs + c * 512 + p * LB::kPiece);
+#pragma unroll
+        for (int r = 0; r < TM; r++) {
+          bf16x8 fa[3];
+#pragma unroll
+          for (int p = 0; p < 3; p++) fa[p] = *reinterpret_cast<const bf16x8*>(as + r * 512 + p * LA::kPiece);
+#pragma unroll
+          for (int q = 0; q < 5; q++)
+#pragma unroll
+            for (int c = 0; c < TN; c++)
+              lo[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kPieceA[q]], fb[c][kPieceB[q]], lo[r][c], 0, 0, 0);
+#pragma unroll
+          for (int c = 0; c < TN; c++)
+            acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[c][0], acc[r][c], 0, 0, 0);
+        }
+        char* nx = smem + ((kt + 1) & 1) * kBuf;
+        sa.template store<CHK>(nx, t, bad);
+        sb.template store<CHK>(nx + LA::kBytes, t, bad);
+        sa.template load<CHK>(lda, kend, t);
+        sb.template load<CHK>(ldb, kend, t);
+        __syncthreads();
+      }
+    };
+    // every row and K slab of the tile in range: no checks
+    if (nk > 0) {
+      if (j.m0 + BMT <= j.m_end && j.n0 + BNT <= g.N && (kend - kbeg) % BK == 0) kloop(std::false_type{});
+      else kloop(std::true_type{});
+    }
+#pragma unroll
+    for (int r = 0; r < TM; r++)
+#pragma unroll
+      for (int c = 0; c < TN; c++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+          acc[r][c][v] = (acc[r][c][v] + lo[r][c][v]) * kSplitDown;
+          bad |= !(fabsf(acc[r][c][v]) <= 3.402823466e38f);
+        }
+  }
+  // a tile with values the split cannot hold, or whose sums left the range
+  if (__syncthreads_or(bad))
+    mainloop_f32<TA, TB, true, WM, WN, TM, TN>(g, j, reinterpret_cast<float*>(smem), acc);
+  store_tile<PLAIN, ACTS>(acc, g, j.C, j.m0 + wm * TM * 32, j.n0 + wn * TN * 32, l32, kh, j.m_end);
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -518,6 +812,64 @@ static int device_cus() {
     cus[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
   }
   return cus[dev];
+}
+
+// The split kernel takes every product of at least kBf3MinK steps that it can
+// read as float4 and whose epilogue it holds.  Transposed both ways (no caller
+// but the entry point), a transposed product with an activation and the
+// general epilogue's activations stay on the fp32 kernel, and so do products
+// that ask for it (GemmArgs::f32).
+// Short K: one MFMA aligns its 16 products to the largest and drops what lies
+// below fp32's last place there.  Over a long sum that is far below the
+// roundings of the sum itself; a short sum with one dominant term is left
+// with about 1.4 x 2^-24 instead of 0.5 (K = 16, lognormal operands: relative
+// error 8.5e-8), and its product is bound by its memory traffic either way.
+constexpr int kBf3MinK = 128;
+static bool bf3_takes(const GemmArgs& g, bool vec, bool plain, bool tA, bool tB) {
+  if (!vec || (tA && tB) || g.f32 || g.K < kBf3MinK) return false;
+  if (g.mode == kEpiAccum || (plain && g.mode == kEpiActGrad)) return true;
+  const unsigned acts = !plain || tA || tB ? kActsNone : g.groups ? kActsMoe : kAllActs;
+  return g.mode == kEpiAct && ((acts >> g.act) & 1);
+}
+
+// ---- which kernel, which tile, how many K chunks --------------------------------
+
+// The split kernel's tiles, by use: 256x128 (8 waves, one workgroup on a CU),
+// 128x128 (4 waves, two on a CU), and for grouped products 128x256.
+enum Bf3Tile : int { kT256x128 = 0, kT128, kTiles };
+
+// Estimated time (us) of M x N x K (x batch) on one tile shape with the K
+// range cut into `splits`: whole rounds of the CUs, each tile with a prologue
+// and epilogue worth ~64 steps of K.  Measured rates (N(0,1) operands): 256x128
+// tiles 210 TFLOP/s, 128x128 190 with two workgroups on a CU and ~130 with
+// one.  The splits' partial sums are written and read once more at ~4 TB/s.
+static double bf3_time(int tile, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t splits, int cus) {
+  const int64_t bm = tile == kT128 ? 128 : 256, bn = 128;
+  const int64_t tiles = ceil_div(M, bm) * ceil_div(N, bn) * batch * splits;
+  const int64_t n = ceil_div(tiles, cus);  // tiles of the busiest CU
+  const double rate = (tile == kT256x128 ? 210. : n >= 2 ? 190. : 130.) * 1e6 / cus;  // FLOP per us and CU
+  const double t = (double)n * 2. * bm * bn * ((double)ceil_div(K, splits) + 64.) / rate;
+  return splits > 1 ? t + 6. + (double)M * N * batch * splits * 8. / 4e6 : t;
+}
+
+struct Bf3Pick {
+  int tile;
+  int64_t splits;
+};
+// The tile with the least estimated time; splits > 0 fixes the K chunks,
+// else up to max_splits are tried.
+static Bf3Pick bf3_pick(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t splits, int64_t max_splits, int cus) {
+  Bf3Pick best{kT128, std::max<int64_t>(splits, 1)};
+  double tb = 1e30;
+  for (int tile = 0; tile < kTiles; tile++)
+    for (int64_t sp = std::max<int64_t>(splits, 1); sp <= std::max<int64_t>(splits > 0 ? splits : max_splits, 1); sp++) {
+      const double t = bf3_time(tile, M, N, K, batch, sp, cus);
+      if (t < tb) {
+        tb = t;
+        best = {tile, sp};
+      }
+    }
+  return best;
 }
 
 int launch_gemm_ex(const GemmArgs& in, bool tA, bool tB, int batch, hipStream_t s) {
@@ -558,40 +910,49 @@ int launch_gemm_ex(const GemmArgs& in, bool tA, bool tB, int batch, hipStream_t 
     set_error("gemm: sign bits need a relu pre-activation / activation pair or a relu gradient, ldmask >= N");
     return -1;
   }
-  // 256-row tiles for large dense plain NN products; 256-column tiles for
-  // the grouped (per-expert) NN products, whose row ranges are short
-  const bool wide = !tA && !tB && vec && plain && !g.groups && !g.kseg && !g.kitems && !g.kchunk && !g.a_rows &&
-                    g.M >= 2048;
-  const bool tallg = !tA && !tB && vec && g.groups && !g.kseg && !g.kitems && !g.kchunk && g.N >= 1024;
-  const int bm = wide ? 2 * BM : BM, bn = tallg ? 2 * BN : BN;
+  const int zs = g.kchunk ? (int)ceil_div(g.K, g.kchunk) : 1;
+  const int cus = device_cus();
+  const bool bf3 = bf3_takes(g, vec, plain, tA, tB);
+  int bm = BM, bn = BN, tile = kT128;
+  if (bf3 && g.groups) {
+    bn = 256;  // 128-row tiles (the caller's tile list), 256 columns
+  } else if (bf3 && plain && !g.kitems && !g.kseg) {
+    tile = bf3_pick(g.M, g.N, g.K, batch, zs, zs, cus).tile;
+    bm = tile == kT128 ? 128 : 256;
+  }
   g.tiles_m = (int)ceil_div(g.M, bm);
   g.tiles_n = (int)ceil_div(g.N, bn);
   // grouped: an upper bound on tile entries, sum_e ceil(n_e / BM) <= M/BM + E
   const int entries = g.groups ? g.tiles_m + g.groups : g.tiles_m;
-  const int zs = g.kchunk ? (int)ceil_div(g.K, g.kchunk) : 1;
-  const dim3 grid(entries * g.tiles_n, batch, zs), block(NT);
-#define NSH_GEMM(TA_, TB_, V_)                                                                        \
-  do {                                                                                               \
-    if (plain) hipLaunchKernelGGL((gemm_f32_kernel<TA_, TB_, V_, true, 1, 1>), grid, block, 0, s, g);  \
-    else hipLaunchKernelGGL((gemm_f32_kernel<TA_, TB_, V_, false, 1, 1>), grid, block, 0, s, g);       \
+  const dim3 grid(entries * g.tiles_n, batch, zs);
+#define NSH_F32(TA_, TB_, V_)                                                                     \
+  do {                                                                                            \
+    if (plain) hipLaunchKernelGGL((gemm_f32_kernel<TA_, TB_, V_, true>), grid, dim3(NT), 0, s, g);  \
+    else hipLaunchKernelGGL((gemm_f32_kernel<TA_, TB_, V_, false>), grid, dim3(NT), 0, s, g);       \
   } while (0)
-  // The 256-row tiles run two workgroups per CU.  When that leaves a
-  // half-full last round but one per CU gives whole rounds (tiles = 256 mod
-  // 512 on 256 CUs, e.g. c5's batched Q/K/V projection: 768 tiles), extra
-  // dynamic LDS holds the kernel to one workgroup per CU (its static 57 KB +
-  // 32 KB > half of the CU's 160 KB): 260 -> 220 us on that projection.
-  // Otherwise two per CU are faster (c5's output layer: 1046 vs 1181 us).
-  const int64_t wide_tiles = (int64_t)entries * g.tiles_n * batch * zs;
-  const int cus = device_cus();
-  const size_t wide_dyn = wide && wide_tiles % (2 * cus) != 0 && wide_tiles % cus == 0 ? 32768 : 0;
-  if (wide) hipLaunchKernelGGL((gemm_f32_kernel<false, false, true, true, 2, 1>), grid, dim3(2 * NT), wide_dyn, s, g);
-  else if (tallg && plain) hipLaunchKernelGGL((gemm_f32_kernel<false, false, true, true, 1, 2>), grid, dim3(2 * NT), 0, s, g);
-  else if (tallg) hipLaunchKernelGGL((gemm_f32_kernel<false, false, true, false, 1, 2>), grid, dim3(2 * NT), 0, s, g);
-  else if (!tA && !tB) { if (vec) NSH_GEMM(false, false, true); else NSH_GEMM(false, false, false); }
-  else if (!tA && tB) { if (vec) NSH_GEMM(false, true, true); else NSH_GEMM(false, true, false); }
-  else if (tA && !tB) { if (vec) NSH_GEMM(true, false, true); else NSH_GEMM(true, false, false); }
-  else { if (vec) NSH_GEMM(true, true, true); else NSH_GEMM(true, true, false); }
-#undef NSH_GEMM
+#define NSH_BF3(TA_, TB_, ACTS_)                                                                              \
+  do {                                                                                                        \
+    if (!plain)                                                                                               \
+      hipLaunchKernelGGL((gemm_bf3_kernel<TA_, TB_, false, kActsNone, 2, 2>), grid, dim3(256), 0, s, g);        \
+    else if (tile == kT256x128)                                                                               \
+      hipLaunchKernelGGL((gemm_bf3_kernel<TA_, TB_, true, ACTS_, 4, 2>), grid, dim3(512), 0, s, g);             \
+    else hipLaunchKernelGGL((gemm_bf3_kernel<TA_, TB_, true, ACTS_, 2, 2>), grid, dim3(256), 0, s, g);          \
+  } while (0)
+  if (bf3 && g.groups) {
+    if (!tB && plain) hipLaunchKernelGGL((gemm_bf3_kernel<false, false, true, kActsMoe, 2, 4>), grid, dim3(512), 0, s, g);
+    else if (!tB) hipLaunchKernelGGL((gemm_bf3_kernel<false, false, false, kActsNone, 2, 4>), grid, dim3(512), 0, s, g);
+    else if (plain) hipLaunchKernelGGL((gemm_bf3_kernel<false, true, true, kActsNone, 2, 4>), grid, dim3(512), 0, s, g);
+    else hipLaunchKernelGGL((gemm_bf3_kernel<false, true, false, kActsNone, 2, 4>), grid, dim3(512), 0, s, g);
+  } else if (bf3) {
+    if (!tA && !tB) NSH_BF3(false, false, kAllActs);
+    else if (!tA) NSH_BF3(false, true, kActsNone);
+    else NSH_BF3(true, false, kActsNone);
+  } else if (!tA && !tB) { if (vec) NSH_F32(false, false, true); else NSH_F32(false, false, false); }
+  else if (!tA && tB) { if (vec) NSH_F32(false, true, true); else NSH_F32(false, true, false); }
+  else if (tA && !tB) { if (vec) NSH_F32(true, false, true); else NSH_F32(true, false, false); }
+  else { if (vec) NSH_F32(true, true, true); else NSH_F32(true, true, false); }
+#undef NSH_F32
+#undef NSH_BF3
   NSH_LAUNCHED();
   return 0;
 }
@@ -624,19 +985,11 @@ static int split_chunk(int K, int splits) { return (int)(ceil_div(ceil_div(K, sp
 
 int gemm_split_count(const GemmArgs& g, int batch) {
   if (!splittable(g) || g.M <= 0 || g.N <= 0 || batch <= 0) return 1;
-  const int64_t tiles = ceil_div(g.M, BM) * ceil_div(g.N, BN) * batch;
-  if (tiles >= 384) return 1;
-  // The largest split (chunks of at least 512) whose workgroups fill whole
-  // rounds of the CUs at up to 4 per CU (c5's output-layer weight gradient,
-  // 256 tiles: 4 chunks, 1016 us against 1032 for 3; its 512 x 512 ones: 32
-  // and 16), else enough chunks for ~768 workgroups.
-  const int cus = device_cus();
-  for (int64_t s = std::min<int64_t>(32, g.K / 512); s >= 2; s--)
-    if (tiles * s <= 4 * cus && (tiles * s) % cus == 0) return (int)ceil_div(g.K, split_chunk(g.K, (int)s));
-  int64_t sp = std::min<int64_t>(ceil_div(768, tiles), g.K / 512);
-  sp = std::min<int64_t>(sp, 32);
-  if (sp < 2) return 1;
-  return (int)ceil_div(g.K, split_chunk(g.K, (int)sp));
+  // chunks of at least 256, at most 32 of them; the estimate prices the
+  // partial sums against the CUs that a few tiles leave idle
+  const int64_t sp =
+      bf3_pick(g.M, g.N, g.K, batch, 0, std::min<int64_t>(32, g.K / 256), device_cus()).splits;
+  return sp < 2 ? 1 : (int)ceil_div(g.K, split_chunk(g.K, (int)sp));
 }
 
 size_t gemm_split_workspace(const GemmArgs& g, int batch, int splits) {

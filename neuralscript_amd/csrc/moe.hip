@@ -797,6 +797,10 @@ static GemmArgs dwg_args(const float* x, const float* dg, float* dWg, int64_t M,
   g.A = x; g.B = dg; g.C = dWg;
   g.M = (int)D; g.N = (int)E; g.K = (int)M;
   g.lda = D; g.ldb = E; g.ldc = E;
+  // dg is zero but for the tokens whose routing is undecided: on bf16 pieces
+  // the largest elements' error grew from 2.0e-5 to 1.5e-4 of the gradient's
+  // rms (4096 tokens, 64 experts), for a product of 0.5 GFLOP
+  g.f32 = true;
   return g;
 }
 
@@ -834,7 +838,12 @@ int launch_moe_backward(const float* x, const float* dout, const float* Wg, cons
   NSH_LAUNCHED();
   // dx = dg Wg^T, then += dH We1[e]^T scattered back to token order
   if (dx) {
-    if (launch_gemm(b.dg, Wg, dx, M, D, E, E, E, D, false, true, 0, s) != 0) return -1;
+    GemmArgs r;
+    r.A = b.dg; r.B = Wg; r.C = dx;
+    r.M = (int)M; r.N = (int)D; r.K = (int)E;
+    r.lda = E; r.ldb = E; r.ldc = D;
+    r.f32 = true;  // as dWg
+    if (launch_gemm_ex(r, false, true, 1, s) != 0) return -1;
     GemmArgs h;
     h.A = b.dH; h.B = We1; h.C = dx;
     h.M = (int)M; h.N = (int)D; h.K = (int)H;

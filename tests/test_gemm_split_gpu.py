@@ -1,0 +1,102 @@
+"""The split (three bf16 pieces) GEMM at the edges of its tiles, against
+float64, and on the values its pieces cannot hold, against the oracle.
+
+Bound of a result: every fp32 rounding of the accumulator is at most 2^-24 of
+the running sum of |a b|, six piece products per 16 of k and one more for each
+K chunk; the three dropped piece products are at most 2^-26 |a b|.
+"""
+import numpy as np
+import pytest
+
+import helpers
+import oracle
+from neuralscript_amd import runtime, synth
+
+pytestmark = pytest.mark.gpu
+
+U = 2.0 ** -24
+
+
+def product(A, B, variant, splits=None, act=0):
+    """C = A . B through the entry point, A [M, K], B [K, N]."""
+    (M, K), N = A.shape, B.shape[1]
+    tA, tB = variant == "tn", variant == "nt"
+    dA = runtime.DeviceArray.from_host(np.ascontiguousarray(A.T if tA else A))
+    dB = runtime.DeviceArray.from_host(np.ascontiguousarray(B.T if tB else B))
+    dC = runtime.DeviceArray(M * N)
+    lda, ldb = M if tA else K, K if tB else N
+    if splits is None:
+        runtime.gemm(dA, dB, dC, M, N, K, lda, ldb, N, tA, tB, act)
+    else:
+        runtime.gemm_splitk(dA, dB, dC, M, N, K, lda, ldb, N, tA, tB, act, splits)
+    return dC.to_host().reshape(M, N)
+
+
+def operands(M, N, K, seed):
+    return (synth.normal(seed, M * K).reshape(M, K), synth.normal(seed + 1, K * N).reshape(K, N))
+
+
+# one element short of, at and past each tile (128 and 256 rows, 128 columns; the
+# contiguous extent of an operand is a multiple of 4), K at the least the split
+# kernel takes and inside a slab, more tiles than CUs
+SHAPES = [(4, 4, 128), (124, 132, 132), (128, 128, 128), (132, 252, 140), (256, 256, 144), (260, 516, 196),
+          (4096, 256, 160), (4100, 4100, 132), (8192, 2052, 128), (260, 132, 124)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("variant", ["nn", "nt", "tn"])
+def test_split_product_against_float64(M, N, K, variant):
+    print(f"split gemm {variant} M={M} N={N} K={K}", flush=True)
+    A, B = operands(M, N, K, M + 3 * N + K)
+    rows = np.unique(np.clip(np.array([0, 1, 31, 32, 127, 128, 255, 256, M // 2, M - 2, M - 1]), 0, M - 1))
+    got = product(A, B, variant)[rows].astype(np.float64)
+    a, b = A[rows].astype(np.float64), B.astype(np.float64)
+    bound = (6 * (K // 16 + 1) + 4) * U * (np.abs(a) @ np.abs(b))
+    assert np.all(np.abs(got - a @ b) <= bound)
+
+
+@pytest.mark.parametrize("M,N,K,splits", [(128, 128, 512, 3), (260, 132, 1032, 4), (512, 512, 4096, 0)])
+@pytest.mark.parametrize("variant", ["nn", "nt", "tn"])
+def test_split_k_product_against_float64(M, N, K, splits, variant):
+    A, B = operands(M, N, K, 7 * M + N + K)
+    got = product(A, B, variant, splits).astype(np.float64)
+    a, b = A.astype(np.float64), B.astype(np.float64)
+    bound = (6 * (K // 16 + 1) + 40) * U * (np.abs(a) @ np.abs(b))
+    assert np.all(np.abs(got - a @ b) <= bound)
+
+
+@pytest.mark.parametrize("M,N,K", [(132, 136, 140), (512, 8192, 128), (8192, 512, 128)])
+@pytest.mark.parametrize("variant", ["nn", "nt", "tn"])
+def test_values_without_three_pieces(M, N, K, variant):
+    """Infinities, NaN and values that bf16 rounds to infinity: where the
+    oracle's are; the rows beside them as if they were not there."""
+    A, B = operands(M, N, K, 11 * M + K)
+    A[1, 0], A[3, K - 1], A[5, 1] = np.inf, -np.inf, np.nan
+    A[6, 0], A[6, 1] = np.inf, -np.inf
+    A[8, 2], A[M - 1, K - 1] = 3.4e38, -3.39e38
+    rows = [0, 1, 2, 3, 4, 5, 6, 7, 8, 9, M - 2, M - 1]
+    with np.errstate(all="ignore"):
+        ref = oracle.matmul(A[rows].ravel(), B.ravel(), len(rows), K, N).reshape(-1, N)
+    got = product(A, B, variant)[rows]
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref))
+    ok = np.isfinite(ref)
+    # (8, .) and (M - 1, .) carry sums of the order of 3e38
+    small = ok & (np.abs(ref) < 1e30)
+    helpers.assert_close(got[small], ref[small], f"beside special values {variant}")
+    assert np.all(np.abs(got[ok] - ref[ok]) <= 1e-5 * np.abs(ref[ok]) + 1e-4)
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -115, 2.0 ** -126, 2.0 ** -135, 2.0 ** -140, 2.0 ** 70])
+@pytest.mark.parametrize("variant", ["nn", "nt", "tn"])
+def test_operands_of_any_magnitude(scale, variant):
+    """Operands down to fp32's subnormals and up to sums past 2^80 keep the
+    relative accuracy of their own bits."""
+    M, N, K = 136, 260, 144
+    A, B = operands(M, N, K, 77)
+    A = (A * np.float32(scale)).astype(np.float32)  # subnormal operands keep the bits fp32 has there
+    B = (B * np.float32(2.0 ** 20)).astype(np.float32)
+    got = product(A, B, variant).astype(np.float64)
+    a, b = A.astype(np.float64), B.astype(np.float64)
+    bound = (K + 8) * U * (np.abs(a) @ np.abs(b)) + 2.0 ** -149 * K
+    assert np.all(np.abs(got - a @ b) <= bound)
