@@ -24,10 +24,9 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "split3.h"
 
 namespace nship {
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 namespace {
 
@@ -134,30 +133,24 @@ __device__ __forceinline__ void score_tile(const float* __restrict__ ks, const f
     }
 }
 
-// Software-pipelined over key tiles: iteration `it` issues the score MFMAs
-// of tile it+1 alongside the softmax of tile it, then O^T += V_it^T P_it^T.
-// LDS holds two K tiles (it+1 in use, the other free for it+2) and two V
-// tiles (it in use, the other free for it+1).  The rescale of O by
+// The key loop in fp32 MFMA, for the workgroups whose Q, K or V the split
+// cannot hold (split3.h): o = unnormalised O^T, m and l the running maximum
+// and sum.  K and V tiles double buffered in LDS.  The rescale of O by
 // exp2(m_old - m_new) is skipped when no lane's running max moved (the factor
 // would be exactly 1).
 template <int DK>
-__global__ __launch_bounds__(kFW * 64) void flash_fwd_kernel(const float* __restrict__ Q, const float* __restrict__ K,
-                                                        const float* __restrict__ V, float* __restrict__ ctx,
-                                                        float* __restrict__ lse, int S, int H, int64_t ld,
-                                                        float scale_log2, int nqb) {
+__device__ __forceinline__ void flash_fwd_f32(const float* __restrict__ Q, const float* __restrict__ K,
+                                              const float* __restrict__ V, float* __restrict__ sm, int S, int64_t ld,
+                                              int hcol, int q0, float scale_log2, floatx16 (&o)[DK / 32], float& m,
+                                              float& l) {
   constexpr int P = DK + 4;
   constexpr int TF = kBK * P;   // floats of one K or V tile in LDS
   constexpr int NDB = DK / 32;  // 32-wide head-dim blocks of the output
-  __shared__ __attribute__((aligned(16))) float sm[4 * TF];
   float* const kbuf = sm;           // K tile i at kbuf + (i & 1) * TF
   float* const vbuf = sm + 2 * TF;  // V tile i at vbuf + (i & 1) * TF
 
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int l32 = lane & 31, kh = lane >> 5;
-  const int L = remap_xcd(blockIdx.x, nqb * H);
-  const int h = L / nqb, q0 = (L % nqb) * (32 * kFW);
-  const int hcol = h * DK;
-  const int qrow = q0 + w * 32 + l32;
+  const int t = threadIdx.x, lane = t & 63;
+  const int l32 = lane & 31, kh = lane >> 5, qrow = q0 + (t >> 6) * 32 + l32;
 
   // B operand of S^T = K Q^T: this lane's query (pre-scaled), head dims 8g + 4kh + (0..3).
   float qf[DK / 2];
@@ -169,12 +162,12 @@ __global__ __launch_bounds__(kFW * 64) void flash_fwd_kernel(const float* __rest
     qf[4 * g + 2] = x.z * scale_log2; qf[4 * g + 3] = x.w * scale_log2;
   }
 
-  floatx16 o[NDB];
 #pragma unroll
   for (int d = 0; d < NDB; d++)
 #pragma unroll
     for (int v = 0; v < 16; v++) o[d][v] = 0.f;
-  float m = -INFINITY, l = 0.f;
+  m = -INFINITY;
+  l = 0.f;
 
   const int nkv = (S + kBK - 1) / kBK;
   HalfTile<DK, kFW * 64> tk, tv;
@@ -182,22 +175,11 @@ __global__ __launch_bounds__(kFW * 64) void flash_fwd_kernel(const float* __rest
   tv.load(V, ld, hcol, 0, S, t);
   tk.store(kbuf, t);
   tv.store(vbuf, t);
-  tk.load(K, ld, hcol, (nkv > 1 ? 1 : 0) * kBK, S, t);
-  tk.store(kbuf + TF, t);
   __syncthreads();
-  floatx16 sc[2], sn[2];
-  score_tile<DK>(kbuf, qf, l32, kh, sc);
-  __syncthreads();  // kbuf tile 0 is overwritten at the end of iteration 0
 
   for (int it = 0; it < nkv; it++) {
-    // prefetch K tile it+2 and V tile it+1 (clamped: the last tiles reload)
-    tk.load(K, ld, hcol, min(it + 2, nkv - 1) * kBK, S, t);
-    tv.load(V, ld, hcol, min(it + 1, nkv - 1) * kBK, S, t);
-    // MFMA bursts run at raised wave priority, so a SIMD's other wave fills
-    // the gaps with its softmax work rather than competing for issue
-    __builtin_amdgcn_s_setprio(1);
-    if (it + 1 < nkv) score_tile<DK>(kbuf + ((it + 1) & 1) * TF, qf, l32, kh, sn);
-    __builtin_amdgcn_s_setprio(0);
+    floatx16 sc[2];
+    score_tile<DK>(kbuf + (it & 1) * TF, qf, l32, kh, sc);
 
     // Online softmax for this lane's query (keys 8*(v/4) + 4kh + v%4 of each block).
     const int kbase = it * kBK;
@@ -239,7 +221,6 @@ __global__ __launch_bounds__(kFW * 64) void flash_fwd_kernel(const float* __rest
     m = mnew;
 
     // O^T += V^T P^T: step s of key block kb pairs key 8*(s/4)+4kh+s%4.
-    __builtin_amdgcn_s_setprio(1);
     const float* vs = vbuf + (it & 1) * TF;
 #pragma unroll
     for (int kb = 0; kb < 2; kb++)
@@ -250,22 +231,348 @@ __global__ __launch_bounds__(kFW * 64) void flash_fwd_kernel(const float* __rest
         for (int d = 0; d < NDB; d++)
           o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vs[key * P + d * 32 + l32], sc[kb][s], o[d], 0, 0, 0);
       }
-    __builtin_amdgcn_s_setprio(0);
 
-    // K tile it (consumed last iteration) and V tile it-1 (consumed last
-    // iteration) are free: fill them with K tile it+2 and V tile it+1.
-    tk.store(kbuf + (it & 1) * TF, t);
+    // (not prefetched: the registers are O's; the last tile reloads)
+    tk.load(K, ld, hcol, min(it + 1, nkv - 1) * kBK, S, t);
+    tv.load(V, ld, hcol, min(it + 1, nkv - 1) * kBK, S, t);
+    tk.store(kbuf + ((it + 1) & 1) * TF, t);
     tv.store(vbuf + ((it + 1) & 1) * TF, t);
     __syncthreads();
-#pragma unroll
-    for (int kb = 0; kb < 2; kb++) sc[kb] = sn[kb];
   }
+}
+
+// One K tile (KT keys x DK) split into pieces on its way to LDS, as the A
+// operand of S^T = K Q^T: [piece][dim / 8][key] chunks of 8 bf16.  NTH
+// threads starting at t = 0, one chunk (8 dims of a key, two float4) each.
+template <int DK, int KT>
+struct KPieces {
+  static constexpr int kItems = KT * DK / 8;
+  static constexpr int kChunk = KT * 16 + (DK == 32 ? 32 : 16);  // spreads a key's chunks over the banks
+  static constexpr int kPiece = DK / 8 * kChunk;
+  static constexpr int kBytes = 3 * kPiece;
+  float v[8];
+  bool in = false;  // the key exists
+  __device__ __forceinline__ void load(const float* __restrict__ X, int64_t ld, int hcol, int key0, int S, int t) {
+    const int key = t / (DK / 8), c = t % (DK / 8);
+    in = key0 + key < S;
+    // wave-uniform tile address + 32-bit offset inside the tile
+    const char* base = reinterpret_cast<const char*>(X + (int64_t)key0 * ld + hcol);
+    const uint32_t off = ((uint32_t)min(key, S - 1 - key0) * (uint32_t)ld + c * 8) * 4u;
+    const float4 a = *reinterpret_cast<const float4*>(base + off);
+    const float4 b = *reinterpret_cast<const float4*>(base + off + 16);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  }
+  __device__ __forceinline__ void store(char* __restrict__ lds, int t, bool& bad) {
+    const int key = t / (DK / 8), c = t % (DK / 8);
+    uint32_t w[3][4];
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = in ? v[j] : 0.f;
+    split_run<8>(v, w[0], w[1], w[2], bad);
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+      *reinterpret_cast<uintx4*>(lds + p * kPiece + c * kChunk + key * 16) = uintx4{w[p][0], w[p][1], w[p][2], w[p][3]};
+  }
+  // A operand: 32 keys from kb * 32, dims 16 g + 8 kh + (0..7)
+  __device__ __forceinline__ static bf16x8 frag(const char* __restrict__ lds, int p, int kb, int g, int l32, int kh) {
+    return *reinterpret_cast<const bf16x8*>(lds + p * kPiece + (2 * g + kh) * kChunk + (kb * 32 + l32) * 16);
+  }
+};
+
+// One tile of KT rows (keys, or queries in the backward) x DK as the operand
+// of a product that contracts over the rows: [piece][chunk of 8 rows][dim].
+// PERM: the rows of a chunk are those that one lane holds of a 32x32
+// accumulator block with those rows (16 s + 4 kh + {0..3, 8..11} of chunk
+// (s, kh) in each 32-row block), so that a probability tile is the other
+// operand straight from its registers; else 8 consecutive rows.
+template <int DK, int KT, bool PERM>
+struct VPieces {
+  static constexpr int kItems = KT * DK / 8;
+  static constexpr int kPiece = KT / 8 * DK * 16;
+  static constexpr int kBytes = 3 * kPiece;
+  float v[8];
+  int lim = 0;  // tile rows below lim exist
+  __device__ __forceinline__ static int row_of(int c, int j) {
+    return PERM ? (c >> 2) * 32 + ((c >> 1) & 1) * 16 + (c & 1) * 4 + (j & 3) + 8 * (j >> 2) : c * 8 + j;
+  }
+  __device__ __forceinline__ void load(const float* __restrict__ X, int64_t ld, int hcol, int row0, int S, int t) {
+    const int c = t / DK, d = t % DK;
+    lim = S - row0;
+    const char* base = reinterpret_cast<const char*>(X + (int64_t)row0 * ld + hcol);
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      v[j] = *reinterpret_cast<const float*>(base + ((uint32_t)min(row_of(c, j), lim - 1) * (uint32_t)ld + d) * 4u);
+  }
+  __device__ __forceinline__ void store(char* __restrict__ lds, int t, bool& bad) {
+    const int c = t / DK, d = t % DK;
+    uint32_t w[3][4];
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = row_of(c, j) < lim ? v[j] : 0.f;
+    split_run<8>(v, w[0], w[1], w[2], bad);
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+      *reinterpret_cast<uintx4*>(lds + p * kPiece + (c * DK + d) * 16) = uintx4{w[p][0], w[p][1], w[p][2], w[p][3]};
+  }
+  // operand: rows of chunk c, dims 32 db + l32
+  __device__ __forceinline__ static bf16x8 frag(const char* __restrict__ lds, int p, int c, int db, int l32) {
+    return *reinterpret_cast<const bf16x8*>(lds + p * kPiece + (c * DK + db * 32 + l32) * 16);
+  }
+};
+
+// 8 fp32 values as the three operand pieces of an MFMA step.
+__device__ __forceinline__ void split8(const float* v, bf16x8 (&f)[3]) {
+  uintx4 w[3];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    uint32_t a, b, c;
+    split_pair(v[2 * j], v[2 * j + 1], a, b, c);
+    w[0][j] = a; w[1][j] = b; w[2][j] = c;
+  }
+#pragma unroll
+  for (int p = 0; p < 3; p++) f[p] = __builtin_bit_cast(bf16x8, w[p]);
+}
+
+// Key tile of the forward: its K and V staging is one chunk per thread each
+// (at head size 32 half the threads stage K, half V).
+template <int DK>
+constexpr int fwd_keys() {
+  return DK == 128 ? 32 : 64;
+}
+
+// S^T tile (KT keys x this wave's 32 queries) = K_tile Q^T, in log2 units
+// (Q is pre-scaled by scale * log2(e)).
+template <int DK, int KT>
+__device__ __forceinline__ void score_pieces(const char* __restrict__ ks, const bf16x8 (&qf)[DK / 16][3], int l32,
+                                             int kh, floatx16 (&sc)[KT / 32]) {
+#pragma unroll
+  for (int kb = 0; kb < KT / 32; kb++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) sc[kb][v] = 0.f;
+  // the leading pieces' products last: the others meet a small accumulator
+  // (gemm.hip: what an MFMA drops is relative to its accumulator)
+#pragma unroll
+  for (int g = 0; g < DK / 16; g++) {
+    bf16x8 f[KT / 32][3];
+#pragma unroll
+    for (int kb = 0; kb < KT / 32; kb++)
+#pragma unroll
+      for (int p = 0; p < 3; p++) f[kb][p] = KPieces<DK, KT>::frag(ks, p, kb, g, l32, kh);
+#pragma unroll
+    for (int q = 0; q < 5; q++)
+#pragma unroll
+      for (int kb = 0; kb < KT / 32; kb++)
+        sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[kb][kPieceA[q]], qf[g][kPieceB[q]], sc[kb], 0, 0, 0);
+  }
+#pragma unroll
+  for (int g = 0; g < DK / 16; g++)
+#pragma unroll
+    for (int kb = 0; kb < KT / 32; kb++)
+      sc[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(KPieces<DK, KT>::frag(ks, 0, kb, g, l32, kh), qf[g][0], sc[kb],
+                                                       0, 0, 0);
+}
+
+// Software-pipelined as flash_fwd_f32, on three-piece bf16 products.  Bound
+// by the matrix cores: 12 MFMAs (32 cycles) per 32 keys x 32 queries x 16
+// dims of both products, against ~15 VALU operations per score for the
+// softmax and the split of P, which the SIMD's other wave hides.
+template <int DK>
+__global__ __launch_bounds__(kFW * 64, 2) void flash_fwd_kernel(const float* __restrict__ Q,
+                                                                const float* __restrict__ K,
+                                                                const float* __restrict__ V, float* __restrict__ ctx,
+                                                                float* __restrict__ lse, int S, int H, int64_t ld,
+                                                                float scale_log2, int nqb) {
+  constexpr int KT = fwd_keys<DK>(), NKB = KT / 32;
+  constexpr int NDB = DK / 32;  // 32-wide head-dim blocks of the output
+  using KP = KPieces<DK, KT>;
+  using VP = VPieces<DK, KT, true>;
+  constexpr int NT = kFW * 64;
+  // at head size 128 the query's pieces and O fill the registers: the scores
+  // of the next tile are not held beside this one's
+  constexpr bool kPipe = DK < 128;
+  constexpr int kAhead = kPipe ? 2 : 1;  // K tiles staged ahead
+  constexpr int kLds = 2 * (KP::kBytes + VP::kBytes);
+  constexpr int kF32 = 4 * kBK * (DK + 4) * 4;  // the fp32 loop's tiles
+  __shared__ __attribute__((aligned(16))) char smem[kLds > kF32 ? kLds : kF32];
+  char* const kbuf = smem;                   // K tile i at kbuf + (i & 1) * KP::kBytes
+  char* const vbuf = smem + 2 * KP::kBytes;  // V tile i at vbuf + (i & 1) * VP::kBytes
+
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int l32 = lane & 31, kh = lane >> 5;
+  const int L = remap_xcd(blockIdx.x, nqb * H);
+  const int h = L / nqb, q0 = (L % nqb) * (32 * kFW);
+  const int hcol = h * DK;
+  const int qrow = q0 + w * 32 + l32;
+
+  floatx16 o[NDB];
+#pragma unroll
+  for (int d = 0; d < NDB; d++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) o[d][v] = 0.f;
+  float m = -INFINITY, l = 0.f;
+  bool bad = false;
+  {
+    // B operand of S^T = K Q^T: this lane's query (pre-scaled), head dims 16 g + 8 kh + (0..7).
+    bf16x8 qf[DK / 16][3];
+#pragma unroll
+    for (int g = 0; g < DK / 16; g++) {
+      const float* p = Q + (int64_t)(qrow < S ? qrow : S - 1) * ld + hcol + 16 * g + 8 * kh;
+      const float4 a = keep4(qrow < S, *reinterpret_cast<const float4*>(p));
+      const float4 b = keep4(qrow < S, *reinterpret_cast<const float4*>(p + 4));
+      float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      uint32_t u[3][4];
+#pragma unroll
+      for (int j = 0; j < 8; j++) x[j] *= scale_log2;
+      split_run<8>(x, u[0], u[1], u[2], bad);
+#pragma unroll
+      for (int p2 = 0; p2 < 3; p2++)
+        qf[g][p2] = __builtin_bit_cast(bf16x8, uintx4{u[p2][0], u[p2][1], u[p2][2], u[p2][3]});
+    }
+    // this thread's staging: a K chunk and a V chunk, or (DK = 32) one of them
+    static_assert(KP::kItems == NT || 2 * KP::kItems == NT, "staging covers the tile");
+    constexpr bool kBoth = KP::kItems == NT;
+    const bool doK = kBoth || t < KP::kItems, doV = kBoth || t >= NT - VP::kItems;
+    const int tv_t = kBoth ? t : t - (NT - VP::kItems);
+    const int nkv = (S + KT - 1) / KT;
+    KP tk;
+    VP tv;
+    auto loadK = [&](int i) { if (doK) tk.load(K, ld, hcol, min(i, nkv - 1) * KT, S, t); };
+    auto loadV = [&](int i) { if (doV) tv.load(V, ld, hcol, min(i, nkv - 1) * KT, S, tv_t); };
+    auto storeK = [&](int i) { if (doK) tk.store(kbuf + (i & 1) * KP::kBytes, t, bad); };
+    auto storeV = [&](int i) { if (doV) tv.store(vbuf + (i & 1) * VP::kBytes, tv_t, bad); };
+    loadK(0);
+    loadV(0);
+    storeK(0);
+    storeV(0);
+    if constexpr (kPipe) {
+      loadK(1);
+      storeK(1);
+    }
+    __syncthreads();
+    floatx16 sc[NKB], sn[kPipe ? NKB : 1];
+    if constexpr (kPipe) {
+      score_pieces<DK, KT>(kbuf, qf, l32, kh, sc);
+      __syncthreads();  // kbuf tile 0 is overwritten at the end of iteration 0
+    }
+
+    for (int it = 0; it < nkv; it++) {
+      // prefetch K tile it+kAhead and V tile it+1 (clamped: the last tiles reload)
+      loadK(it + kAhead);
+      loadV(it + 1);
+      // MFMA bursts run at raised wave priority, so a SIMD's other wave fills
+      // the gaps with its softmax work rather than competing for issue
+      __builtin_amdgcn_s_setprio(1);
+      if constexpr (!kPipe) score_pieces<DK, KT>(kbuf + (it & 1) * KP::kBytes, qf, l32, kh, sc);
+      else if (it + 1 < nkv) score_pieces<DK, KT>(kbuf + ((it + 1) & 1) * KP::kBytes, qf, l32, kh, sn);
+      __builtin_amdgcn_s_setprio(0);
+
+      // Online softmax for this lane's query (keys 8*(v/4) + 4kh + v%4 of each block).
+      const int kbase = it * KT;
+      if (kbase + KT > S) {
+#pragma unroll
+        for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+          for (int v = 0; v < 16; v++) {
+            const int key = kbase + kb * 32 + 8 * (v >> 2) + 4 * kh + (v & 3);
+            if (key >= S) sc[kb][v] = -INFINITY;
+          }
+      }
+      float mloc = -INFINITY;
+#pragma unroll
+      for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) mloc = fmaxf(mloc, sc[kb][v]);
+      mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+      const float mnew = fmaxf(m, mloc);
+      if (__any(mnew > m)) {
+        const float corr = exp2_hw(m - mnew);
+        l *= corr;
+#pragma unroll
+        for (int d = 0; d < NDB; d++)
+#pragma unroll
+          for (int v = 0; v < 16; v++) o[d][v] *= corr;
+      }
+      float lsum = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+          const float p = exp2_hw(sc[kb][v] - mnew);
+          sc[kb][v] = p;
+          lsum += p;
+        }
+      lsum += __shfl_xor(lsum, 32, 64);
+      l += lsum;
+      m = mnew;
+
+      // K tile it (it - 1 unpipelined) and V tile it-1, consumed last
+      // iteration, are free: fill them with K tile it+2 (it+1) and V tile it+1 (here, so
+      // that the staging registers are not held over the products).
+      storeK(it + kAhead);
+      storeV(it + 1);
+
+      // O^T += V^T P^T, 32 keys at a time: this lane's scores 8 s .. 8 s + 7
+      // of key block kb are the operand of step s (VPieces' PERM order).  The
+      // 32 keys are summed apart, leading pieces last, and then added to O:
+      // O would otherwise be rounded, and its operands truncated to its last
+      // place, 6 S / 16 times.
+      const char* vs = vbuf + (it & 1) * VP::kBytes;
+#pragma unroll
+      for (int kb = 0; kb < NKB; kb++) {
+        bf16x8 pf[2][3];
+#pragma unroll
+        for (int s2 = 0; s2 < 2; s2++) {
+          float x[8];
+#pragma unroll
+          for (int j = 0; j < 8; j++) x[j] = sc[kb][8 * s2 + j];
+          split8(x, pf[s2]);
+        }
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int d = 0; d < NDB; d++) {
+          floatx16 part;
+#pragma unroll
+          for (int v = 0; v < 16; v++) part[v] = 0.f;
+#pragma unroll
+          for (int s2 = 0; s2 < 2; s2++) {
+            bf16x8 vf[3];
+#pragma unroll
+            for (int p = 0; p < 3; p++) vf[p] = VP::frag(vs, p, kb * 4 + s2 * 2 + kh, d, l32);
+#pragma unroll
+            for (int q = 0; q < 5; q++)
+              part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[kPieceA[q]], pf[s2][kPieceB[q]], part, 0, 0, 0);
+          }
+#pragma unroll
+          for (int s2 = 0; s2 < 2; s2++)
+            part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(VP::frag(vs, 0, kb * 4 + s2 * 2 + kh, d, l32), pf[s2][0],
+                                                           part, 0, 0, 0);
+#pragma unroll
+          for (int v = 0; v < 16; v++) o[d][v] += part[v];
+          // (head size 128: operands read ahead across blocks would spill)
+          if constexpr (DK == 128) __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+      }
+
+      __syncthreads();
+      if constexpr (kPipe) {
+#pragma unroll
+        for (int kb = 0; kb < NKB; kb++) sc[kb] = sn[kb];
+      }
+    }
+  }
+  // values the split cannot hold, or sums that left the range
+  bad |= !(l <= 3.402823466e38f);
+#pragma unroll
+  for (int d = 0; d < NDB; d++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) bad |= !(fabsf(o[d][v]) <= 3.402823466e38f);
+  float* const sm = reinterpret_cast<float*>(smem);
+  if (__syncthreads_or(bad)) flash_fwd_f32<DK>(Q, K, V, sm, S, ld, hcol, q0, scale_log2, o, m, l);
 
   // Row statistics for the backward pass: log2-sum-exp of the scaled scores.
   if (lse && kh == 0 && qrow < S) lse[(int64_t)h * S + qrow] = m + log2f(l);
 
   // O^T (d, query) / l  ->  LDS [query][d]  ->  coalesced rows of ctx.
-  static_assert(kFW * 32 * (DK + 1) <= 4 * TF, "output staging fits the K/V buffers");
+  static_assert(kFW * 32 * (DK + 1) * 4 <= (int)sizeof(smem), "output staging fits the K/V buffers");
   const float inv = 1.f / l;
   float* T = sm + w * 32 * (DK + 1);
 #pragma unroll
