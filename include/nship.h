@@ -215,9 +215,9 @@ int nsh_op_attention_fwd(const float* Q, const float* K, const float* V, float* 
  * head the gradient of softmax(Q K^T / sqrt(D/H)) V; the core of the
  * ATTENTION_GRAD_* kernels, codegen.cpp:1785-1907.  workspace: bytes from
  * nsh_op_attention_bwd_workspace(S, D, H, store_ds).  store_ds != 0 keeps dS
- * (H*S*S floats, when S % 64 == 0 and the head size is 32 or 64) so that dQ
- * is one product over it instead of a pass that recomputes S and dP; the
- * result is the same to fp32 rounding. */
+ * (H * S * S floats, its rows rounded up to a multiple of 64, for head sizes
+ * up to 128 and up to 16 GiB) so that dQ is one product over it instead of a
+ * pass that recomputes S and dP; the result is the same to fp32 rounding. */
 size_t nsh_op_attention_bwd_workspace(int64_t S, int64_t D, int64_t H, int store_ds);
 int nsh_op_attention_bwd(const float* Q, const float* K, const float* V, const float* O, const float* dO,
                          const float* lse, float* dQ, float* dK, float* dV, int64_t S, int64_t D, int64_t H,

@@ -36,7 +36,7 @@ __device__ __forceinline__ float4 keep4(bool keep, float4 x) {
   return make_float4(keep ? x.x : 0.f, keep ? x.y : 0.f, keep ? x.z : 0.f, keep ? x.w : 0.f);
 }
 
-constexpr int kBQ = 128;  // queries (keys) per workgroup of the backward kernels
+constexpr int kBQ = 128;  // queries per workgroup of the backward's dQ kernels
 constexpr int kFW = 8;     // forward: waves per workgroup (32 queries each), sharing every K/V tile
 constexpr int kBK = 64;   // keys per tile
 
@@ -631,11 +631,11 @@ __global__ __launch_bounds__(256) void attn_unpad_kernel(const float* __restrict
 //    transposed layout (lane = query): dS^T feeds dQ^T = K^T dS^T.
 // ============================================================================
 
-template <int DK>
+template <int DK, int NTH>
 struct QTile {  // one 64-query tile of Q and dO (row pitch P) plus lse, delta
   static constexpr int P = DK + 4;
   static constexpr int kFloats = 2 * 64 * P + 128;
-  static constexpr int kPer = 64 * DK / 4 / 256;  // float4 per thread per matrix
+  static constexpr int kPer = 64 * DK / 4 / NTH;  // float4 per thread per matrix
   float4 q[kPer], g[kPer];
   float l = 0.f, d = 0.f;
   int lim = 0;  // tile rows below lim exist
@@ -646,7 +646,7 @@ struct QTile {  // one 64-query tile of Q and dO (row pitch P) plus lse, delta
     lim = S - q0;
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
-      const int idx = t + 256 * i;
+      const int idx = t + NTH * i;
       const int r = idx / (DK / 4), c = (idx % (DK / 4)) * 4;
       const int64_t row = r < lim ? q0 + r : S - 1;
       q[i] = *reinterpret_cast<const float4*>(Q + row * ld + hcol + c);
@@ -662,7 +662,7 @@ struct QTile {  // one 64-query tile of Q and dO (row pitch P) plus lse, delta
   __device__ void store(float* __restrict__ sm, int t) const {
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
-      const int idx = t + 256 * i;
+      const int idx = t + NTH * i;
       const int r = idx / (DK / 4), c = (idx % (DK / 4)) * 4;
       *reinterpret_cast<float4*>(sm + r * P + c) = keep4(r < lim, q[i]);
       *reinterpret_cast<float4*>(sm + 64 * P + r * P + c) = keep4(r < lim, g[i]);
@@ -674,18 +674,326 @@ struct QTile {  // one 64-query tile of Q and dO (row pitch P) plus lse, delta
   }
 };
 
-// STORE_DS: also write dS = P o (dP - delta) (unscaled) to dS[h][query][key]
-// for flash_bwd_dq_ds_kernel; requires S % 64 == 0.
-// Two workgroups per CU up to DK = 64; at DK = 128 a lane's K and V rows and
-// its dK / dV accumulators (4 x DK/2 registers) need one wave per SIMD.
+// dS of one lane's 16 accumulator rows of the 32-query block from q0 to
+// dS[h][query][key], row pitch ldds (S rounded up to the dQ pass's key tile:
+// the keys past S in it are written as the zeros they are).  Lanes 0-31 /
+// 32-63 write 32 consecutive keys of one query row each; the rows' addresses
+// are wave-uniform, 4 ldds + key a 32-bit offset.
+__device__ __forceinline__ void store_ds_rows(const floatx16& x, float* __restrict__ dS, int64_t hS, int q0, int key,
+                                              int kh, int S, int64_t ldds) {
+  if (key >= ldds) return;
+  char* row = reinterpret_cast<char*>(dS + (hS + q0) * ldds);
+  const uint32_t off = ((uint32_t)(4 * kh) * (uint32_t)ldds + (uint32_t)key) * 4u;
+  if (q0 + 32 <= S) {
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        *reinterpret_cast<float*>(row + (8 * g + j) * ldds * 4 + off) = x[4 * g + j];
+  } else {
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        if (q0 + 4 * kh + 8 * g + j < S) *reinterpret_cast<float*>(row + (8 * g + j) * ldds * 4 + off) = x[4 * g + j];
+  }
+}
+
+// A probability tile's way from the wave that made it to its partner: 16
+// accumulators per lane as four float4.
+__device__ __forceinline__ void put_block(float* __restrict__ buf, int lane, const floatx16& x) {
+#pragma unroll
+  for (int g = 0; g < 4; g++)
+    *reinterpret_cast<float4*>(buf + (g * 64 + lane) * 4) = make_float4(x[4 * g], x[4 * g + 1], x[4 * g + 2], x[4 * g + 3]);
+}
+// x = P o (x - delta), P from put_block, delta of the block's 32 queries.
+__device__ __forceinline__ void take_ds(const float* __restrict__ buf, const float* __restrict__ delta, int lane,
+                                        int kh, floatx16& x) {
+#pragma unroll
+  for (int g = 0; g < 4; g++) {
+    const float4 p = *reinterpret_cast<const float4*>(buf + (g * 64 + lane) * 4);
+    const float4 d = *reinterpret_cast<const float4*>(delta + 8 * g + 4 * kh);
+    x[4 * g] = p.x * (x[4 * g] - d.x);
+    x[4 * g + 1] = p.y * (x[4 * g + 1] - d.y);
+    x[4 * g + 2] = p.z * (x[4 * g + 2] - d.z);
+    x[4 * g + 3] = p.w * (x[4 * g + 3] - d.w);
+  }
+}
+// x = P = 2^(c x - lse); keys past the end: exponent -inf (kneg), P = 0; lse
+// is finite or +inf, so no NaN, and no per-element branch.
+__device__ __forceinline__ void take_p(const float* __restrict__ lse, int kh, float c_log2, float kneg, floatx16& x) {
+#pragma unroll
+  for (int v = 0; v < 16; v++) x[v] = exp2_hw(fmaf(x[v], c_log2, kneg) - lse[8 * (v >> 2) + 4 * kh + (v & 3)]);
+}
+
+constexpr int kPW = 4;             // backward dK / dV: wave pairs per workgroup, 32 keys each
+constexpr int kPNT = 128 * kPW;    // its threads
+
+// The query loop in fp32 MFMA, for the workgroups whose operands the split
+// cannot hold; waves, roles and outputs as in flash_bwd_dkdv_kernel.
 template <int DK, bool STORE_DS>
-__global__ __launch_bounds__(256, DK >= 128 ? 1 : 2) void flash_bwd_dkdv_kernel(const float* __restrict__ Q, const float* __restrict__ K,
+__device__ __forceinline__ void flash_bwd_dkdv_f32(const float* __restrict__ Q, const float* __restrict__ X,
+                                                   const float* __restrict__ dO, const float* __restrict__ lse,
+                                                   const float* __restrict__ delta, float* __restrict__ dS,
+                                                   float* __restrict__ sm, int S, int h, int key, int role,
+                                                   int64_t ld, float c_log2, int64_t ldds,
+                                                   floatx16 (&acc)[DK / 32]) {
+  using Tile = QTile<DK, kPNT>;
+  constexpr int NDB = DK / 32;
+  const int t = threadIdx.x, lane = t & 63, l32 = lane & 31, kh = lane >> 5;
+  const int hcol = h * DK;
+  const float kneg = key < S ? 0.f : -INFINITY;
+  float* pbuf = sm + Tile::kFloats + ((t >> 6) % kPW) * 1024;
+  float xf[DK / 2];  // K or V row of this lane's key, head dims 8g + 4kh + (0..3)
+#pragma unroll
+  for (int g = 0; g < DK / 8; g++) {
+    const float4 a = keep4(key < S, *reinterpret_cast<const float4*>(X + (int64_t)(key < S ? key : S - 1) * ld + hcol + 8 * g + 4 * kh));
+    xf[4 * g] = a.x; xf[4 * g + 1] = a.y; xf[4 * g + 2] = a.z; xf[4 * g + 3] = a.w;
+  }
+#pragma unroll
+  for (int d = 0; d < NDB; d++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[d][v] = 0.f;
+  const float* rows = sm + (role ? 64 * Tile::P : 0);  // S from Q rows, dP from dO rows
+  const float* cols = sm + (role ? 0 : 64 * Tile::P);  // dV from dO, dK from Q
+  const float* ls = sm + 2 * 64 * Tile::P;
+  for (int it = 0; it < (S + 63) / 64; it++) {
+    {
+      Tile tile;
+      tile.load(Q, dO, lse, delta, ld, hcol, h * S, it * 64, S, t);
+      tile.store(sm, t);
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int qb = 0; qb < 2; qb++) {
+      floatx16 x;
+#pragma unroll
+      for (int v = 0; v < 16; v++) x[v] = 0.f;
+#pragma unroll
+      for (int g = 0; g < DK / 8; g++) {
+        const float4 a = *reinterpret_cast<const float4*>(rows + (qb * 32 + l32) * Tile::P + 8 * g + 4 * kh);
+        x = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, xf[4 * g + 0], x, 0, 0, 0);
+        x = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, xf[4 * g + 1], x, 0, 0, 0);
+        x = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, xf[4 * g + 2], x, 0, 0, 0);
+        x = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, xf[4 * g + 3], x, 0, 0, 0);
+      }
+      if (!role) {
+        take_p(ls + qb * 32, kh, c_log2, kneg, x);
+        put_block(pbuf, lane, x);
+      }
+      __syncthreads();
+      if (role) {
+        take_ds(pbuf, ls + 64 + qb * 32, lane, kh, x);
+        if constexpr (STORE_DS) store_ds_rows(x, dS, (int64_t)h * S, it * 64 + qb * 32, key, kh, S, ldds);
+      }
+      // step s pairs query 8(s/4) + 4kh + s%4
+#pragma unroll
+      for (int s2 = 0; s2 < 16; s2++) {
+        const int qr = qb * 32 + 8 * (s2 >> 2) + 4 * kh + (s2 & 3);
+#pragma unroll
+        for (int d = 0; d < NDB; d++)
+          acc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s2], cols[qr * Tile::P + d * 32 + l32], acc[d], 0, 0, 0);
+      }
+      __syncthreads();
+    }
+  }
+}
+
+// Staging of a role's half of one 32-query tile: `rows` (Q or dO) as the rows
+// of its scores' product (KPieces), `cols` (the other) as the contraction of
+// its sum (VPieces), `stat` (lse or delta) of the queries.  4 DK chunks of 8
+// floats each, over the role's 256 threads: at head size 32 half of them
+// stage rows, half columns.
+template <int DK>
+struct RolePieces {
+  using KP = KPieces<DK, 32>;
+  using VP = VPieces<DK, 32, true>;
+  static constexpr int kNT = kPNT / 2;
+  static_assert(KP::kItems == kNT || 2 * KP::kItems == kNT, "chunks divide evenly");
+  static constexpr bool kBoth = KP::kItems == kNT;
+  static constexpr int kV = KP::kBytes, kStat = kV + VP::kBytes, kBytes = kStat + 128;
+  KP k;
+  VP v;
+  float st = 0.f;
+  // stat of a query past the end: `past` (lse = +inf makes P = 0 there)
+  __device__ __forceinline__ void load(const float* __restrict__ rows, const float* __restrict__ cols,
+                                       const float* __restrict__ stat, float past, int64_t ld, int hcol, int q0, int S,
+                                       int t) {
+    if (kBoth || t < KP::kItems) k.load(rows, ld, hcol, q0, S, t);
+    if (kBoth || t >= KP::kItems) v.load(cols, ld, hcol, q0, S, kBoth ? t : t - KP::kItems);
+    if (t < 32) st = q0 + t < S ? stat[q0 + t] : past;
+  }
+  __device__ __forceinline__ void store(char* __restrict__ lds, int t, bool& bad) {
+    if (kBoth || t < KP::kItems) k.store(lds, t, bad);
+    if (kBoth || t >= KP::kItems) v.store(lds + kV, kBoth ? t : t - KP::kItems, bad);
+    if (t < 32) reinterpret_cast<float*>(lds + kStat)[t] = st;
+  }
+};
+
+// acc[d] += A^T B over 32 queries: A = 16 accumulator values of this lane (its
+// key's P or dS), B = columns of a VPieces tile.  Summed apart, leading pieces
+// last, as the forward's P V.
+template <int DK>
+__device__ __forceinline__ void add_outer(const floatx16& a, const char* __restrict__ lds, int l32, int kh,
+                                          floatx16 (&acc)[DK / 32]) {
+  using VP = VPieces<DK, 32, true>;
+  bf16x8 f[2][3];
+#pragma unroll
+  for (int s2 = 0; s2 < 2; s2++) {
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) x[j] = a[8 * s2 + j];
+    split8(x, f[s2]);
+  }
+#pragma unroll
+  for (int d = 0; d < DK / 32; d++) {
+    floatx16 part;
+#pragma unroll
+    for (int v = 0; v < 16; v++) part[v] = 0.f;
+#pragma unroll
+    for (int s2 = 0; s2 < 2; s2++) {
+      bf16x8 b[3];
+#pragma unroll
+      for (int p = 0; p < 3; p++) b[p] = VP::frag(lds, p, s2 * 2 + kh, d, l32);
+#pragma unroll
+      for (int q = 0; q < 5; q++)
+        part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[s2][kPieceA[q]], b[kPieceB[q]], part, 0, 0, 0);
+    }
+#pragma unroll
+    for (int s2 = 0; s2 < 2; s2++)
+      part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[s2][0], VP::frag(lds, 0, s2 * 2 + kh, d, l32), part, 0, 0, 0);
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[d][v] += part[v];
+  }
+}
+
+// dK and dV: one workgroup per 128 keys, 32-query tiles of Q and dO through
+// LDS, every product on three-piece bf16.  A pair of waves shares 32 keys
+// (lane = key): the first (role 0) forms S and P and sums dV += P^T dO, the
+// second (role 1) forms dP, takes P through LDS, and sums dK += dS^T Q.  Each
+// so holds the pieces of one row of K or V and one accumulator (both would not
+// fit the registers), and the pair sits on one SIMD (waves w and w + 4), one
+// wave's softmax and splitting under the other's MFMAs.  Role 1 works one tile
+// behind role 0, each role staging the operands it reads itself, so that one
+// barrier a tile orders both P and the staging (with both roles on one tile
+// and a barrier between P and dS, c5's pass took 8.0 ms).
+// 4 S^2 D products at 6 MFMA passes.
+// STORE_DS: also write dS = P o (dP - delta) (unscaled) for
+// flash_bwd_dq_ds_kernel.
+template <int DK, bool STORE_DS>  // DK 32 or 64
+__global__ __launch_bounds__(kPNT, 2) void flash_bwd_dkdv_kernel(
+    const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
+    const float* __restrict__ dO, const float* __restrict__ lse, const float* __restrict__ delta,
+    float* __restrict__ dK, float* __restrict__ dV, float* __restrict__ dS, int S, int H, int64_t ld, float scale,
+    float c_log2, int nkb, int64_t ldds) {
+  constexpr int NDB = DK / 32;
+  using Tile = RolePieces<DK>;
+  constexpr int kF32 = QTile<DK, kPNT>::kFloats * 4 + kPW * 4096;
+  constexpr int kP = 4 * Tile::kBytes;           // P tiles: two per pair
+  constexpr int kLds = kP + 2 * kPW * 4096;
+  __shared__ __attribute__((aligned(16))) char smem[kLds > kF32 ? kLds : kF32];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int l32 = lane & 31, kh = lane >> 5;
+  const int role = __builtin_amdgcn_readfirstlane(w / kPW);
+  const int L = remap_xcd(blockIdx.x, nkb * H);
+  const int h = L / nkb, k0 = (L % nkb) * (32 * kPW) + (w % kPW) * 32;
+  const int hcol = h * DK;
+  const int64_t hS = (int64_t)h * S;
+  const int key = k0 + l32;  // this lane's key (column of S)
+  const float* __restrict__ X = role ? V : K;
+
+  floatx16 acc[NDB];
+#pragma unroll
+  for (int d = 0; d < NDB; d++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[d][v] = 0.f;
+  bool bad = false;
+  {
+    const float kneg = key < S ? 0.f : -INFINITY;
+    char* const mine = smem + role * 2 * Tile::kBytes;  // this role's two tiles
+    float* const pbuf = reinterpret_cast<float*>(smem + kP) + (w % kPW) * 2048;
+    const int tr = t % Tile::kNT;
+    // B operand: the K or V row of this lane's key, head dims 16 g + 8 kh + (0..7).
+    bf16x8 xf[DK / 16][3];
+#pragma unroll
+    for (int g = 0; g < DK / 16; g++) {
+      const float* p = X + (int64_t)(key < S ? key : S - 1) * ld + hcol + 16 * g + 8 * kh;
+      const float4 a = keep4(key < S, *reinterpret_cast<const float4*>(p));
+      const float4 b = keep4(key < S, *reinterpret_cast<const float4*>(p + 4));
+      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      uint32_t u[3][4];
+      split_run<8>(x, u[0], u[1], u[2], bad);
+#pragma unroll
+      for (int q = 0; q < 3; q++) xf[g][q] = __builtin_bit_cast(bf16x8, uintx4{u[q][0], u[q][1], u[q][2], u[q][3]});
+    }
+    Tile tile;
+    const int nq = (S + 31) / 32;
+    const float* __restrict__ rows = role ? dO : Q;
+    const float* __restrict__ cols = role ? Q : dO;
+    const float* __restrict__ stat = (role ? delta : lse) + hS;
+    const float past = role ? 0.f : INFINITY;
+    tile.load(rows, cols, stat, past, ld, hcol, 0, S, tr);
+    tile.store(mine, tr, bad);
+    __syncthreads();
+    for (int step = 0; step <= nq; step++) {
+      const int it = step - role;  // this role's tile
+      if (it >= 0 && it < nq) {    // (uniform per wave)
+        const char* cur = mine + (it & 1) * Tile::kBytes;
+        tile.load(rows, cols, stat, past, ld, hcol, min(it + 1, nq - 1) * 32, S, tr);  // (the last tile reloads)
+        // element v: query 8(v/4) + 4kh + v%4, key = this lane's
+        floatx16 x[1];
+        __builtin_amdgcn_s_setprio(1);
+        score_pieces<DK, 32>(cur, xf, l32, kh, x);
+        __builtin_amdgcn_s_setprio(0);
+        const float* st = reinterpret_cast<const float*>(cur + Tile::kStat);
+        if (!role) {
+          take_p(st, kh, c_log2, kneg, x[0]);
+          put_block(pbuf + (it & 1) * 1024, lane, x[0]);
+        } else {
+          take_ds(pbuf + (it & 1) * 1024, st, lane, kh, x[0]);
+          if constexpr (STORE_DS) store_ds_rows(x[0], dS, hS, it * 32, key, kh, S, ldds);
+        }
+        // the next tile, here so that its registers are not held over the products
+        tile.store(mine + ((it + 1) & 1) * Tile::kBytes, tr, bad);
+        __builtin_amdgcn_s_setprio(1);
+        add_outer<DK>(x[0], cur + Tile::kV, l32, kh, acc);
+        __builtin_amdgcn_s_setprio(0);
+      }
+      __syncthreads();
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < NDB; d++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) bad |= !(fabsf(acc[d][v]) <= 3.402823466e38f);
+  if (__syncthreads_or(bad))
+    flash_bwd_dkdv_f32<DK, STORE_DS>(Q, X, dO, lse, delta, dS, reinterpret_cast<float*>(smem), S, h, key, role, ld,
+                                     c_log2, ldds, acc);
+  // accumulator v of block d: key 8(v/4) + 4kh + v%4 of the pair's, head dim d*32 + l32
+  float* __restrict__ out = role ? dK : dV;
+  const float f = role ? scale : 1.f;
+#pragma unroll
+  for (int d = 0; d < NDB; d++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+      const int kr = k0 + 8 * (v >> 2) + 4 * kh + (v & 3);
+      if (kr < S) out[(int64_t)kr * ld + hcol + d * 32 + l32] = acc[d][v] * f;
+    }
+}
+
+// dK and dV at head size 128, in fp32 MFMA: one workgroup per 128 keys (32 per
+// wave), 64-query tiles; P and dS are the A operands of both sums straight
+// from registers.  (On bf16 pieces one row of K or V and one accumulator take
+// 160 registers a lane there, and the rest of the loop does not fit beside
+// them.)  One wave per SIMD: a lane holds its K and V rows and dK, dV.
+template <int DK, bool STORE_DS>
+__global__ __launch_bounds__(256, 1) void flash_bwd_dkdv_f32_kernel(const float* __restrict__ Q, const float* __restrict__ K,
                                                              const float* __restrict__ V, const float* __restrict__ dO,
                                                              const float* __restrict__ lse,
                                                              const float* __restrict__ delta, float* __restrict__ dK,
                                                              float* __restrict__ dV, float* __restrict__ dS, int S,
-                                                             int H, int64_t ld, float scale, float c_log2, int nkb) {
-  using Tile = QTile<DK>;
+                                                             int H, int64_t ld, float scale, float c_log2, int nkb, int64_t ldds) {
+  using Tile = QTile<DK, 256>;
   constexpr int NDB = DK / 32;
   __shared__ __attribute__((aligned(16))) float sm[2 * Tile::kFloats];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -757,21 +1065,7 @@ __global__ __launch_bounds__(256, DK >= 128 ? 1 : 2) void flash_bwd_dkdv_kernel(
         sc[v] = p;
         dp[v] = p * (dp[v] - ds[qr]);
       }
-      if (STORE_DS && key < S) {
-        // lanes 0-31 / 32-63 write 32 consecutive keys of one query row each;
-        // every query row of the tile exists (S % 64 == 0)
-        // element v sits in row 8 (v / 4) + v % 4: walk a single pointer
-        float* __restrict__ dst = dS + ((int64_t)h * S + it * 64 + qb * 32 + 4 * kh) * S + key;
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            *dst = dp[4 * g + j];
-            dst += S;
-          }
-          dst += 4 * (int64_t)S;
-        }
-      }
+      if constexpr (STORE_DS) store_ds_rows(dp, dS, hS, it * 64 + qb * 32, key, kh, S, ldds);
       __builtin_amdgcn_s_setprio(1);
       // dV += P^T dO, dK += dS^T Q: step s pairs query 8(s/4) + 4kh + s%4.
 #pragma unroll
@@ -901,24 +1195,27 @@ __global__ __launch_bounds__(256) void flash_bwd_dq_kernel(const float* __restri
   }
 }
 
-// dQ = scale * dS K from the stored dS (S % 64 == 0): the dq kernel's
-// transposed product dQ^T += K^T dS^T without recomputing S and dP.  Lane =
+// dQ = scale * dS K from the stored dS: the dq kernel's transposed product
+// dQ^T += K^T dS^T without recomputing S and dP, on three-piece bf16.  Lane =
 // query; its dS operands of a 64-key tile are 8 float4 read straight from its
-// row, dlo/dhi[j] = keys key0 + 32 kb + 8 j + 4 kh + (0..3) for kb = 0/1
-// (drow includes the 4 kh offset; a lane past the end reads row S - 1 and its
-// operands are zeroed where they are taken).  Each half is reloaded for the
-// next tile as soon as its MFMAs have taken it, and each K tile (float4 i of
-// thread t: key (t + 256 i) / (DK/4), dims 4 ((t + 256 i) % (DK/4))) is
-// loaded an iteration before it is written to LDS, so both prefetches cross
-// the loop's back edge and the compiler cannot sink them next to their use.
+// row (pitch ldds, a multiple of 64; a lane past the end reads row S - 1 and
+// its operands are zeroed where they are taken), keys key0 + 16 step + 8 kh +
+// (0..7) for MFMA step `step`.  Each 32-key half is reloaded for the next
+// tile as soon as it is split, and each K tile is loaded an iteration before
+// it is written to LDS, so both prefetches cross the loop's back edge and the
+// compiler cannot sink them next to their use.  Bound by HBM: dS is read once
+// (8.6 GB at 16384 tokens and 8 heads).
 template <int DK>
-__global__ __launch_bounds__(256) void flash_bwd_dq_ds_kernel(const float* __restrict__ K,
-                                                              const float* __restrict__ dS, float* __restrict__ dQ,
-                                                              int S, int H, int64_t ld, float scale, int nqb) {
+__global__ __launch_bounds__(256, 2) void flash_bwd_dq_ds_kernel(const float* __restrict__ K,
+                                                                 const float* __restrict__ dS,
+                                                                 float* __restrict__ dQ, int S, int H, int64_t ld,
+                                                                 float scale, int nqb, int64_t ldds) {
   constexpr int NDB = DK / 32;
-  constexpr int P = DK + 4;
-  constexpr int kPer = kBK * DK / 4 / 256;
-  __shared__ __attribute__((aligned(16))) float sm[2 * kBK * P > 4 * 32 * (DK + 1) ? 2 * kBK * P : 4 * 32 * (DK + 1)];
+  using VP = VPieces<DK, kBK, false>;
+  constexpr int kIt = VP::kItems / 256;
+  constexpr int kOut = 4 * 32 * (DK + 1) * 4, kF32 = kBK * (DK + 4) * 4;
+  constexpr int kLds = 2 * VP::kBytes > kOut ? 2 * VP::kBytes : kOut;
+  __shared__ __attribute__((aligned(16))) char smem[kLds > kF32 ? kLds : kF32];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int l32 = lane & 31, kh = lane >> 5;
   const int L = remap_xcd(blockIdx.x, nqb * H);
@@ -926,79 +1223,126 @@ __global__ __launch_bounds__(256) void flash_bwd_dq_ds_kernel(const float* __res
   const int hcol = h * DK;
   const int qrow = q0 + w * 32 + l32;
   const bool qin = qrow < S;
-  const float* __restrict__ drow = dS + ((int64_t)h * S + (qin ? qrow : S - 1)) * S + 4 * kh;
+  const float* __restrict__ drow = dS + ((int64_t)h * S + (qin ? qrow : S - 1)) * ldds + 8 * kh;
   floatx16 acc[NDB];
 #pragma unroll
   for (int d = 0; d < NDB; d++)
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[d][v] = 0.f;
+  const int nkv = (S + kBK - 1) / kBK;
+  bool bad = false;
+  {
+    VP kt[kIt];
+    // native vectors: an array of HIP float4 carried across the loop stays in
+    // scratch memory, these stay in registers
+    fvec4 dlo[4], dhi[4];
+    auto load_k = [&](int i) {
+#pragma unroll
+      for (int j = 0; j < kIt; j++) kt[j].load(K, ld, hcol, min(i, nkv - 1) * kBK, S, t + 256 * j);
+    };
+    auto store_k = [&](char* __restrict__ ks) {
+#pragma unroll
+      for (int j = 0; j < kIt; j++) kt[j].store(ks, t + 256 * j, bad);
+    };
+    auto load_d = [&](fvec4(&dd)[4], int key0) {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        dd[j] = *reinterpret_cast<const fvec4*>(drow + key0 + 16 * (j >> 1) + 4 * (j & 1));
+    };
+    // the MFMAs of one 32-key half (steps 2 kb, 2 kb + 1 of the tile)
+    auto half = [&](const char* __restrict__ ks, fvec4(&dd)[4], int kb, int next) {
+      bf16x8 f[2][3];
+#pragma unroll
+      for (int s2 = 0; s2 < 2; s2++) {
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = qin ? dd[2 * s2 + (j >> 2)][j & 3] : 0.f;
+        split8(x, f[s2]);
+      }
+      load_d(dd, next + 32 * kb);
+      __builtin_amdgcn_sched_barrier(0);  // issue the reload before the MFMAs
+#pragma unroll
+      for (int d = 0; d < NDB; d++) {
+        floatx16 part;
+#pragma unroll
+        for (int v = 0; v < 16; v++) part[v] = 0.f;
+#pragma unroll
+        for (int s2 = 0; s2 < 2; s2++) {
+          bf16x8 b[3];
+#pragma unroll
+          for (int p = 0; p < 3; p++) b[p] = VP::frag(ks, p, kb * 4 + s2 * 2 + kh, d, l32);
+#pragma unroll
+          for (int q = 0; q < 5; q++)
+            part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[kPieceA[q]], f[s2][kPieceB[q]], part, 0, 0, 0);
+        }
+#pragma unroll
+        for (int s2 = 0; s2 < 2; s2++)
+          part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(VP::frag(ks, 0, kb * 4 + s2 * 2 + kh, d, l32), f[s2][0], part,
+                                                         0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[d][v] += part[v];
+      }
+    };
 
-  // native vectors: an array of HIP float4 carried across the loop stays in
-  // scratch memory, these stay in registers
-  fvec4 kt[kPer];
-  float4 dlo[4], dhi[4];
-  auto load_k = [&](int key0) {
-#pragma unroll
-    for (int i = 0; i < kPer; i++) {
-      const int idx = t + 256 * i;
-      kt[i] = *reinterpret_cast<const fvec4*>(K + (int64_t)(key0 + idx / (DK / 4)) * ld + hcol + (idx % (DK / 4)) * 4);
-    }
-  };
-  auto store_k = [&](float* __restrict__ ks) {
-#pragma unroll
-    for (int i = 0; i < kPer; i++) {
-      const int idx = t + 256 * i;
-      *reinterpret_cast<fvec4*>(ks + (idx / (DK / 4)) * P + (idx % (DK / 4)) * 4) = kt[i];
-    }
-  };
-  auto load_d = [&](float4(&dd)[4], int key0) {
-#pragma unroll
-    for (int j = 0; j < 4; j++) dd[j] = *reinterpret_cast<const float4*>(drow + key0 + 8 * j);
-  };
-  // the MFMAs of one 32-key half: step s pairs key 32 kb + 8 (s/4) + 4 kh + s%4
-  auto half = [&](const float* __restrict__ ks, float4(&dd)[4], int kb, int next) {
-    float dv[16];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const float4 x = keep4(qin, dd[j]);
-      dv[4 * j] = x.x; dv[4 * j + 1] = x.y; dv[4 * j + 2] = x.z; dv[4 * j + 3] = x.w;
-    }
-    load_d(dd, next + 32 * kb);
-    __builtin_amdgcn_sched_barrier(0);  // issue the reload before the MFMAs
-#pragma unroll
-    for (int s2 = 0; s2 < 16; s2++) {
-      const int kr = kb * 32 + 8 * (s2 >> 2) + 4 * kh + (s2 & 3);
-#pragma unroll
-      for (int d = 0; d < NDB; d++)
-        acc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(ks[kr * P + d * 32 + l32], dv[s2], acc[d], 0, 0, 0);
-    }
-  };
-
-  const int nkv = S / kBK;
-  load_k(0);
-  store_k(sm);
-  // the loop's issue order (K tile, then the two halves), so that each wait
-  // in the loop covers only the loads it needs
-  load_k((nkv > 1 ? 1 : 0) * kBK);
-  load_d(dlo, 0);
-  load_d(dhi, 32);
-  __syncthreads();
-  for (int it = 0; it < nkv; it++) {
-    const int cur = it & 1;
-    // K tile it+1 (loaded an iteration ago) into the buffer that the last
-    // iteration read; the barrier at this iteration's end publishes it.  The
-    // last iteration stores a tile that nothing reads.
-    store_k(sm + (cur ^ 1) * kBK * P);
-    load_k(min(it + 2, nkv - 1) * kBK);
-    __builtin_amdgcn_sched_barrier(0);
-    const int next = min(it + 1, nkv - 1) * kBK;  // the last step reloads its own tile
-    const float* ks = sm + cur * kBK * P;
-    half(ks, dlo, 0, next);
-    half(ks, dhi, 1, next);
+    load_k(0);
+    store_k(smem);
+    // the loop's issue order (K tile, then the two halves), so that each wait
+    // in the loop covers only the loads it needs
+    load_k(1);
+    load_d(dlo, 0);
+    load_d(dhi, 32);
     __syncthreads();
+    for (int it = 0; it < nkv; it++) {
+      const int cur = it & 1;
+      // K tile it+1 (loaded an iteration ago) into the buffer that the last
+      // iteration read; the barrier at this iteration's end publishes it.  The
+      // last iteration stores a tile that nothing reads.
+      store_k(smem + (cur ^ 1) * VP::kBytes);
+      load_k(it + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      const int next = min(it + 1, nkv - 1) * kBK;  // the last step reloads its own tile
+      const char* ks = smem + cur * VP::kBytes;
+      half(ks, dlo, 0, next);
+      half(ks, dhi, 1, next);
+      __syncthreads();
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < NDB; d++)
+#pragma unroll
+    for (int v = 0; v < 16; v++) bad |= !(fabsf(acc[d][v]) <= 3.402823466e38f);
+  if (__syncthreads_or(bad)) {
+    // K values the split cannot hold, or a dS that is not finite: fp32 MFMA
+    constexpr int P = DK + 4;
+    float* ks = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int d = 0; d < NDB; d++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[d][v] = 0.f;
+    for (int it = 0; it < nkv; it++) {
+      for (int i = t; i < kBK * DK; i += 256) {
+        const int key = it * kBK + i / DK;
+        ks[(i / DK) * P + i % DK] = key < S ? K[(int64_t)key * ld + hcol + i % DK] : 0.f;
+      }
+      __syncthreads();
+#pragma unroll 1
+      for (int kb = 0; kb < 2; kb++) {
+#pragma unroll
+        for (int s2 = 0; s2 < 16; s2++) {
+          // step s2 pairs key 32 kb + 16 (s2 / 8) + 8 kh + s2 % 8
+          const int kr = kb * 32 + 16 * (s2 >> 3) + (s2 & 7);
+          const float x = qin ? drow[it * kBK + kr] : 0.f;
+#pragma unroll
+          for (int d = 0; d < NDB; d++)
+            acc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(ks[(kr + 8 * kh) * P + d * 32 + l32], x, acc[d], 0, 0, 0);
+        }
+      }
+      __syncthreads();
+    }
   }
   // dQ^T (d, query) -> LDS [query][d] -> rows of dQ
-  float* T = sm + w * 32 * (DK + 1);
+  __syncthreads();  // the tiles are read; T takes their place
+  float* T = reinterpret_cast<float*>(smem) + w * 32 * (DK + 1);
 #pragma unroll
   for (int d = 0; d < NDB; d++)
 #pragma unroll
@@ -1446,11 +1790,14 @@ int launch_attention_fwd(const float* Q, const float* K, const float* V, float* 
   return unpad_copy(Op, ctx, ld, S, H, DK, dkp, s);
 }
 
+// Row pitch of dS: S rounded up to the dQ pass's key tile.
+static int64_t ds_pitch(int64_t S) { return ceil_div(S, kBK) * kBK; }
+
 size_t attention_bwd_ds_floats(int64_t S, int64_t D, int64_t H) {
-  if (S <= 0 || H <= 0 || D % H != 0 || S % kBK != 0 || !padded_dk(D / H)) return 0;
-  const double bytes = 4.0 * (double)H * (double)S * (double)S;
+  if (S <= 0 || H <= 0 || D % H != 0 || !padded_dk(D / H)) return 0;
+  const double bytes = 4.0 * (double)H * (double)S * (double)ds_pitch(S);
   if (bytes > 16.0 * 1024 * 1024 * 1024) return 0;  // recompute beyond 16 GiB
-  return (size_t)(H * S * S);
+  return (size_t)(H * S * ds_pitch(S));
 }
 
 // The backward kernels of one tile width on arrays of row pitch ld.
@@ -1463,17 +1810,31 @@ static int flash_bwd(const float* Q, const float* K, const float* V, const float
                      (int)S, (int)H, ld);
   NSH_LAUNCHED();
   const int nb = (int)ceil_div(S, kBQ);
+  static_assert(32 * kPW == kBQ, "the dK / dV kernels take 128 keys a workgroup");
   const dim3 grid(nb * (unsigned)H), block(256);
-  if (ds_ws) {
-    hipLaunchKernelGGL((flash_bwd_dkdv_kernel<DK, true>), grid, block, 0, s, Q, K, V, dO, lse, delta, dK, dV, ds_ws,
-                       (int)S, (int)H, ld, scale, cl2, nb);
-    hipLaunchKernelGGL(flash_bwd_dq_ds_kernel<DK>, grid, block, 0, s, K, ds_ws, dQ, (int)S, (int)H, ld, scale, nb);
+  const int64_t ldds = ds_ws ? ds_pitch(S) : 0;
+  if constexpr (DK == 128) {
+    if (ds_ws)
+      hipLaunchKernelGGL((flash_bwd_dkdv_f32_kernel<DK, true>), grid, block, 0, s, Q, K, V, dO, lse, delta, dK, dV,
+                         ds_ws, (int)S, (int)H, ld, scale, cl2, nb, ldds);
+    else
+      hipLaunchKernelGGL((flash_bwd_dkdv_f32_kernel<DK, false>), grid, block, 0, s, Q, K, V, dO, lse, delta, dK, dV,
+                         nullptr, (int)S, (int)H, ld, scale, cl2, nb, ldds);
   } else {
-    hipLaunchKernelGGL((flash_bwd_dkdv_kernel<DK, false>), grid, block, 0, s, Q, K, V, dO, lse, delta, dK, dV,
-                       nullptr, (int)S, (int)H, ld, scale, cl2, nb);
+    if (ds_ws)
+      hipLaunchKernelGGL((flash_bwd_dkdv_kernel<DK, true>), grid, dim3(kPNT), 0, s, Q, K, V, dO, lse, delta, dK, dV,
+                         ds_ws, (int)S, (int)H, ld, scale, cl2, nb, ldds);
+    else
+      hipLaunchKernelGGL((flash_bwd_dkdv_kernel<DK, false>), grid, dim3(kPNT), 0, s, Q, K, V, dO, lse, delta, dK, dV,
+                         nullptr, (int)S, (int)H, ld, scale, cl2, nb, ldds);
+  }
+  NSH_LAUNCHED();
+  if (ds_ws)
+    hipLaunchKernelGGL(flash_bwd_dq_ds_kernel<DK>, grid, block, 0, s, K, ds_ws, dQ, (int)S, (int)H, ld, scale, nb,
+                       ldds);
+  else
     hipLaunchKernelGGL(flash_bwd_dq_kernel<DK>, grid, block, 0, s, Q, K, V, dO, lse, delta, dQ, (int)S, (int)H, ld,
                        scale, cl2, nb);
-  }
   NSH_LAUNCHED();
   return 0;
 }

@@ -585,13 +585,13 @@ struct Bf3Stage {
   static constexpr int NC = BK / W;             // W-chunks of a slab
   static constexpr int kN = ROWS * NC / NTH;    // chunks per thread
   static_assert(kN >= 1 && kN * NTH == ROWS * NC, "the chunks divide evenly");
-  float v[kN][W];
+  float v[2][kN][W];   // two slabs in flight (even, odd)
   const float* p[kN];  // chunk i of slab 0: its row (in range), or (KC false) the tile's first row
   uint32_t ro[kN];     // KC false: byte offset of chunk i's row (in range) from there
   unsigned rin;        // bit i set: the row of chunk i is in range
   int64_t off, wrap;   // of the next slab; what the end of a K block adds
   int k, inblk, kblk;  // next slab, its place in its K block, the block's length
-  int lim;             // k of the held slab below lim exist
+  int lim[2];          // k of the held slabs below lim exist
 
   __device__ __forceinline__ static void pos(int idx, int& r, int& kc) {
     // (KC false: ROWS is a multiple of the wave, so kc is uniform and the
@@ -624,11 +624,11 @@ struct Bf3Stage {
     wrap = kb > 0 ? sk - kb * unit : 0;
     off = (kb > 0 ? kbeg / kb * wrap : 0) + kbeg * unit;
   }
-  // The next slab, then on by one; past the last one (k >= kend - BK) it stays
-  // (nothing reads the slab then loaded again).
-  template <bool CHK>
+  // The next slab into set Z, then on by one; past the last one (k >= kend -
+  // BK) it stays (nothing reads the slab then loaded again).
+  template <bool CHK, int Z>
   __device__ __forceinline__ void load(int64_t ld, int kend, int t) {
-    lim = kend - k;
+    lim[Z] = kend - k;
 #pragma unroll
     for (int i = 0; i < kN; i++) {
       int r, kc;
@@ -637,16 +637,16 @@ struct Bf3Stage {
 #pragma unroll
         for (int u = 0; u < W; u += 4) {
           // (whole float4: kend and k are multiples of 4)
-          const int ku = CHK ? min(kc * W + u, lim - 4) : kc * W + u;
+          const int ku = CHK ? min(kc * W + u, lim[Z] - 4) : kc * W + u;
           const float4 x = *reinterpret_cast<const float4*>(p[i] + off + ku);
-          v[i][u] = x.x; v[i][u + 1] = x.y; v[i][u + 2] = x.z; v[i][u + 3] = x.w;
+          v[Z][i][u] = x.x; v[Z][i][u + 1] = x.y; v[Z][i][u + 2] = x.z; v[Z][i][u + 3] = x.w;
         }
       } else {
         const float* q = p[i] + off;
 #pragma unroll
         for (int u = 0; u < W; u++) {
-          if (CHK) q = p[i] + off + (int64_t)min(u, lim - 1 - kc * W) * ld;
-          v[i][u] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(q) + ro[i]);
+          if (CHK) q = p[i] + off + (int64_t)min(u, lim[Z] - 1 - kc * W) * ld;
+          v[Z][i][u] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(q) + ro[i]);
           if (!CHK) q += ld;
         }
       }
@@ -659,7 +659,7 @@ struct Bf3Stage {
     off += next ? wrap : 0;
     inblk = next ? 0 : inblk;
   }
-  template <bool CHK>
+  template <bool CHK, int Z>
   __device__ __forceinline__ void store(char* __restrict__ lds, int t, bool& bad) {
     using L = Bf3Layout<ROWS>;
 #pragma unroll
@@ -669,10 +669,10 @@ struct Bf3Stage {
       uint32_t w0[W / 2], w1[W / 2], w2[W / 2];
 #pragma unroll
       for (int u = 0; u < W; u++) {
-        if (CHK) v[i][u] = ((rin >> i) & 1) && kc * W + u < lim ? v[i][u] : 0.f;
-        v[i][u] *= kSplitUp;
+        if (CHK) v[Z][i][u] = ((rin >> i) & 1) && kc * W + u < lim[Z] ? v[Z][i][u] : 0.f;
+        v[Z][i][u] *= kSplitUp;
       }
-      split_run<W>(v[i], w0, w1, w2, bad);
+      split_run<W>(v[Z][i], w0, w1, w2, bad);
       if constexpr (W == 8) {
         char* d = lds + kc * L::kHalf + r * 16;
         *reinterpret_cast<uintx4*>(d) = uintx4{w0[0], w0[1], w0[2], w0[3]};
@@ -709,8 +709,10 @@ constexpr unsigned kActsMoe = 1u << kActId | 1u << kActGeluMoe;
 // 4096 x 4096 runs at 216 (fp32 MFMA 127), 16384 x 512 x 8192 at 203 (126).
 // 64x64 per wave is what two accumulators leave room for at two waves per
 // SIMD; 128x64 per wave with one accumulator ran at 234, with the error above.
-// The slab after next is loaded right after its registers were split and
-// stored, so a load has a whole slab of MFMAs to arrive.
+// Two slabs of loads are in flight: a load has two slabs of MFMAs to arrive
+// (one: 1500 us on that product against 1390, 197 against 184 on 16384 x 512 x
+// 2048, same box).  Measured and not kept: the two waves of a SIMD taking turns
+// at the matrix core, one barrier per turn (1475 us).
 template <bool TA, bool TB, bool PLAIN, unsigned ACTS, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf3_kernel(GemmArgs g) {
   constexpr int TM = 2, TN = 2;
@@ -738,41 +740,56 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf3_kernel(GemmArgs g) {
       Bf3Stage<TB, BNT, NTT> sb;
       sa.init(j.A, lda, j.m0, j.m_end, kbeg, t, g.a_rows, g.kblk, g.sAk);
       sb.init(j.B, ldb, j.n0, g.N, kbeg, t, nullptr, g.kblk, g.sBk);
-      sa.template load<CHK>(lda, kend, t);
-      sb.template load<CHK>(ldb, kend, t);
-      sa.template store<CHK>(smem, t, bad);
-      sb.template store<CHK>(smem + LA::kBytes, t, bad);
-      sa.template load<CHK>(lda, kend, t);
-      sb.template load<CHK>(ldb, kend, t);
+      auto load = [&](auto z) {
+        constexpr int Z = decltype(z)::value;
+        sa.template load<CHK, Z>(lda, kend, t);
+        sb.template load<CHK, Z>(ldb, kend, t);
+      };
+      auto store = [&](auto z, char* __restrict__ to) {
+        constexpr int Z = decltype(z)::value;
+        sa.template store<CHK, Z>(to, t, bad);
+        sb.template store<CHK, Z>(to + LA::kBytes, t, bad);
+      };
+      using Even = std::integral_constant<int, 0>;
+      using Odd = std::integral_constant<int, 1>;
+      load(Even{});
+      load(Odd{});
+      store(Even{}, smem);
+      load(Even{});
       __syncthreads();
-      for (int kt = 0; kt < nk; kt++) {
+      // slab kt; slab kt + 1 (set z) to LDS, slab kt + 3 into its registers
+      auto slab = [&](int kt, auto z) {
         const char* as = smem + (kt & 1) * kBuf + kh * LA::kHalf + (wm * TM * 32 + l32) * 16;
         const char* bs = smem + (kt & 1) * kBuf + LA::kBytes + kh * LB::kHalf + (wn * TN * 32 + l32) * 16;
-        bf16x8 fb[TN][3];
+        char* nx = smem + ((kt + 1) & 1) * kBuf;
+        bf16x8 fa[TM][3], fb[TN][3];
 #pragma unroll
         for (int c = 0; c < TN; c++)
 #pragma unroll
           for (int p = 0; p < 3; p++) fb[c][p] = *reinterpret_cast<const bf16x8*>(bs + c * 512 + p * LB::kPiece);
 #pragma unroll
-        for (int r = 0; r < TM; r++) {
-          bf16x8 fa[3];
+        for (int r = 0; r < TM; r++)
 #pragma unroll
-          for (int p = 0; p < 3; p++) fa[p] = *reinterpret_cast<const bf16x8*>(as + r * 512 + p * LA::kPiece);
+          for (int p = 0; p < 3; p++) fa[r][p] = *reinterpret_cast<const bf16x8*>(as + r * 512 + p * LA::kPiece);
+#pragma unroll
+        for (int r = 0; r < TM; r++) {
 #pragma unroll
           for (int q = 0; q < 5; q++)
 #pragma unroll
             for (int c = 0; c < TN; c++)
-              lo[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kPieceA[q]], fb[c][kPieceB[q]], lo[r][c], 0, 0, 0);
+              lo[r][c] =
+                  __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[r][kPieceA[q]], fb[c][kPieceB[q]], lo[r][c], 0, 0, 0);
 #pragma unroll
           for (int c = 0; c < TN; c++)
-            acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[0], fb[c][0], acc[r][c], 0, 0, 0);
+            acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[r][0], fb[c][0], acc[r][c], 0, 0, 0);
         }
-        char* nx = smem + ((kt + 1) & 1) * kBuf;
-        sa.template store<CHK>(nx, t, bad);
-        sb.template store<CHK>(nx + LA::kBytes, t, bad);
-        sa.template load<CHK>(lda, kend, t);
-        sb.template load<CHK>(ldb, kend, t);
+        store(z, nx);
+        load(z);
         __syncthreads();
+      };
+      for (int kt = 0; kt < nk; kt += 2) {
+        slab(kt, Odd{});
+        if (kt + 1 < nk) slab(kt + 1, Even{});
       }
     };
     // every row and K slab of the tile in range: no checks

@@ -671,8 +671,9 @@ int attention_backward(ns_model* m, Frame& fr, const Instr& I, AttnGrads* out) {
   {
     Prof p(m, "attention_bwd");
     const size_t nds = attention_bwd_ds_floats(BS, D, H);
+    // no room for dS: the pass that recomputes S and dP for dQ
     float* ds = nds ? scratch(m, "attn_ds", nds) : nullptr;
-    if (nds && !ds) return -1;
+    if (nds && !ds) (void)hipGetLastError();
     const void* rd[5] = {sv.qkv, sv.qkv + BS * D, sv.qkv + 2 * BS * D, sv.ctx, dPre};
     float* pad = nullptr;
     if (!attention_in_place(D, H, D, rd, 5) && !(pad = scratch(m, "attn_pad", attention_pad_floats(BS, D, H, true))))

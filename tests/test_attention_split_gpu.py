@@ -89,3 +89,82 @@ def test_forward_values_of_any_magnitude(scale):
     got, _ = core(Q, K, V, H)
     ref = reference(Q, K, V, H)
     assert np.max(np.abs(got - ref)) <= bar(S, ref) + 2.0 ** -149 * S
+
+
+def gradients(Q, K, V, dO, H, store_ds=1):
+    S, D = Q.shape
+    gQ, gK, gV, gdO = (DA.from_host(a) for a in (Q, K, V, dO))
+    ctx, lse = DA(S * D), DA(S * H)
+    runtime.op("attention_fwd", gQ, gK, gV, ctx, lse, S, D, H)
+    out = [DA(S * D) for _ in range(3)]
+    nb = runtime.lib().nsh_op_attention_bwd_workspace(S, D, H, store_ds)
+    ws = DA.from_host(np.full(nb // 4 + 1, np.nan, np.float32))  # what the pass leaves unwritten must not be read
+    runtime.op("attention_bwd", gQ, gK, gV, ctx, gdO, lse, *out, S, D, H, store_ds, ws)
+    return [o.to_host().reshape(S, D) for o in out]
+
+
+def reference_gradients(Q, K, V, dO, H):
+    Q, K, V, dO = (a.astype(np.float64) for a in (Q, K, V, dO))
+    dQ, dK, dV = (np.zeros(Q.shape) for _ in range(3))
+    sc = 1.0 / np.sqrt(np.float64(Q.shape[1] // H))
+    for h in range(H):
+        p, c = probabilities(Q, K, H, h)
+        with np.errstate(all="ignore"):
+            dV[:, c] = p.T @ dO[:, c]
+            dp = dO[:, c] @ V[:, c].T
+            ds = p * (dp - np.sum(p * dp, axis=1, keepdims=True))
+            dQ[:, c], dK[:, c] = ds @ K[:, c] * sc, ds.T @ Q[:, c] * sc
+    return dQ, dK, dV
+
+
+def gradient_bounds(Q, K, V, dO, H):
+    """The same sums over absolute values, dP - rowsum(P dP) as |dP| +
+    rowsum(P |dP|) (it may cancel): a score's error is at most 2^-24 (6 dk / 16
+    + 8) |q| |k| / sqrt(dk), which a probability takes over relatively, and
+    every later sum adds less than that again."""
+    Q, K, V, dO = (np.abs(a.astype(np.float64)) for a in (Q, K, V, dO))
+    dk = Q.shape[1] // H
+    return Q, K, V, dO, 2.0 ** -24 * (6 * dk / 16 + 8) * np.sqrt(dk), 1.0 / np.sqrt(np.float64(dk))
+
+
+def assert_gradients(arrs, H, got):
+    Qa, Ka, Va, dOa, unit, sc = gradient_bounds(*arrs, H)
+    refs = reference_gradients(*arrs, H)
+    for h in range(H):
+        p, c = probabilities(arrs[0], arrs[1], H, h)
+        dp = dOa[:, c] @ Va[:, c].T
+        ds = p * (dp + np.sum(p * dp, axis=1, keepdims=True)) * sc
+        for g, r, most in zip(got, refs, (ds @ Ka[:, c], ds.T @ Qa[:, c], p.T @ dOa[:, c])):
+            assert np.all(np.abs(g[:, c] - r[:, c]) <= unit * most)
+
+
+# one short of and one past the query tile (32), the dQ pass's key tile (64)
+# and a workgroup's keys (128); with and without the stored dS
+@pytest.mark.parametrize("S", [1, 31, 33, 63, 65, 127, 129, 300])
+@pytest.mark.parametrize("dk", [32, 64, 128])
+@pytest.mark.parametrize("store_ds", [0, 1])
+def test_gradient_tile_edges(S, dk, store_ds):
+    print(f"attention gradients S={S} dk={dk} store_ds={store_ds}", flush=True)
+    H = 2
+    arrs = inputs(S, H * dk, 17 * S + dk, 4)
+    assert_gradients(arrs, H, gradients(*arrs, H, store_ds))
+
+
+@pytest.mark.parametrize("dk", [32, 64])
+def test_gradients_of_values_without_three_pieces(dk):
+    """A value near fp32's largest, an infinite one or a NaN in one row: where
+    float64's gradients are finite the results follow them, where they are
+    not the results are not finite either."""
+    S, H = 200, 2
+    base = inputs(S, H * dk, 3, 4)
+    for which, value in [(3, 3.39e38), (3, np.inf), (3, np.nan), (2, np.nan)]:
+        arrs = [a.copy() for a in base]
+        arrs[which][9, 2] = value
+        print(f"attention gradients dk={dk} operand {which} = {value}", flush=True)
+        got, ref = gradients(*arrs, H), reference_gradients(*arrs, H)
+        other = slice(dk, 2 * dk)  # the second head holds no special value
+        clean = reference_gradients(*base, H)
+        for g, r, c in zip(got, ref, clean):
+            assert np.max(np.abs(g[:, other] - c[:, other])) <= bar(S, c[:, other])
+            assert not np.any(np.isfinite(g[:, :dk][~np.isfinite(r[:, :dk])]) &
+                              (np.abs(g[:, :dk][~np.isfinite(r[:, :dk])]) < 1e30))
