@@ -7,7 +7,7 @@
 // (CUDA counterparts ns_gemm_kernel / ns_grad_a_kernel / ns_grad_w_kernel,
 // /root/reference/src/codegen/cuda_backend.cpp:58-79, 446-467.)
 //
-// Design (wave64).  Two kernels, one set of operand modes and epilogues:
+// Design (wave64).  Three kernels, one set of operand modes and epilogues:
 //  * gemm_bf3_kernel (16-byte aligned operands): fp32 products as six bf16
 //    MFMAs over three-piece operands (split3.h).  Operands are read as fp32,
 //    split in registers on their way to LDS, and each K slab of 16 is held
@@ -15,7 +15,9 @@
 //    order for either memory order of the operand (8 consecutive k of one row
 //    per lane), read back as conflict-free float4s.
 //  * gemm_f32_kernel (any alignment): fp32 MFMA 32x32x2, 128x128 tiles.
-//  * Both: K advances in 16-wide slabs staged in LDS, double buffered, one
+//  * gemm_small_kernel: products of a few tiles, whose K is dealt out to the
+//    waves of a workgroup.
+//  * The first two: K advances in 16-wide slabs staged in LDS, double buffered, one
 //    barrier per slab, global loads in flight under the MFMAs; workgroup ids
 //    are remapped so each XCD (ids are dealt round-robin over the 8 XCDs)
 //    owns a contiguous run of tiles, grouped 8 tile-rows at a time for L2
@@ -813,6 +815,159 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_bf3_kernel(GemmArgs g) {
   store_tile<PLAIN, ACTS>(acc, g, j.C, j.m0 + wm * TM * 32, j.n0 + wn * TN * 32, l32, kh, j.m_end);
 }
 
+// ---- products too small for the tiled kernels ------------------------------------
+
+// Few output tiles leave most CUs idle and every K slab of the tiled kernels
+// waits for its loads (about 1 us a slab with one workgroup on a CU).  Here a
+// workgroup takes 32 TM x 32 outputs, its 8 waves deal out the 16-steps of K,
+// each loading its operands straight into registers, kSmallU steps at a time
+// and without barriers, and the eight partial sums meet in LDS.  Bound by the
+// memory traffic (each workgroup reads its 32 columns of B once, and A through
+// L2) and, below a few microseconds, by its one or two round trips.
+constexpr int kSmallW = 8;  // waves, each every 8th step of K
+constexpr int kSmallU = 4;  // steps of loads in flight per wave
+
+// One 32 x 16 operand step in registers: this lane's row, 8 consecutive k.
+template <bool KC>
+struct SmallStep {
+  float v[8];
+  // row: this lane's (in range), k: first of its 8; kend: the contraction's end
+  __device__ __forceinline__ void load(const float* __restrict__ base, int64_t ld, int64_t row, int64_t kb, int k,
+                                       int kloc, int kend) {
+    if (KC) {
+      const float* p = base + row * ld + kb;
+#pragma unroll
+      for (int u = 0; u < 8; u += 4) {
+        // (whole float4: kend is a multiple of 4)
+        const bool in = k + u < kend;
+        const float4 x = *reinterpret_cast<const float4*>(p + (in ? kloc + u : 0));
+        v[u] = in ? x.x : 0.f; v[u + 1] = in ? x.y : 0.f; v[u + 2] = in ? x.z : 0.f; v[u + 3] = in ? x.w : 0.f;
+      }
+    } else {
+      const float* p = base + row + kb;
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const bool in = k + u < kend;
+        const float x = p[(int64_t)(in ? kloc + u : 0) * ld];
+        v[u] = in ? x : 0.f;
+      }
+    }
+  }
+};
+
+// PIECES: three-piece bf16 with two accumulators, as gemm_bf3_kernel; else, and
+// for what the pieces cannot hold, fp32 MFMA (step j of a 16-step pairs k = j
+// and 8 + j).  Epilogue: kEpiAct (with the pre-activation / activation pair),
+// kEpiActGrad from aux, kEpiAccum.
+template <bool TA, bool TB, bool PIECES, int TM>
+__global__ __launch_bounds__(64 * kSmallW, 2) void gemm_small_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) float part[kSmallW][TM * 32 * 32];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, l32 = lane & 31, kh = lane >> 5;
+  const int M = g.M, N = g.N, K = g.K;
+  const int m0 = (int)(blockIdx.x / g.tiles_n) * 32 * TM, n0 = (int)(blockIdx.x % g.tiles_n) * 32;
+  const float* __restrict__ A = g.A + (int64_t)blockIdx.y * g.sA;
+  const float* __restrict__ B = g.B + (int64_t)blockIdx.y * g.sB;
+  int64_t ra[TM];
+#pragma unroll
+  for (int r = 0; r < TM; r++) ra[r] = min(m0 + r * 32 + l32, M - 1);
+  const int64_t rb = min(n0 + l32, N - 1);
+  const int steps = (K + 15) / 16;
+  floatx16 acc[TM];
+  bool bad = false;
+  auto run = [&](auto pieces) {
+    constexpr bool P3 = decltype(pieces)::value;
+    floatx16 lo[TM];
+#pragma unroll
+    for (int r = 0; r < TM; r++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) { acc[r][v] = 0.f; lo[r][v] = 0.f; }
+    for (int s0 = w; s0 < steps; s0 += kSmallW * kSmallU) {
+      SmallStep<!TA> a[kSmallU][TM];
+      SmallStep<TB> b[kSmallU];
+#pragma unroll
+      for (int u = 0; u < kSmallU; u++) {
+        if (s0 + u * kSmallW >= steps) break;  // (uniform)
+        const int k = (s0 + u * kSmallW) * 16 + 8 * kh;
+        const int blk = g.kblk ? k / g.kblk : 0, kloc = g.kblk ? k % g.kblk : k;
+        const bool in = k < K;  // (not for the upper half of a last step of 8)
+#pragma unroll
+        for (int r = 0; r < TM; r++) a[u][r].load(A, g.lda, ra[r], in ? blk * g.sAk : 0, k, kloc, K);
+        b[u].load(B, g.ldb, rb, in ? blk * g.sBk : 0, k, kloc, K);
+      }
+#pragma unroll
+      for (int u = 0; u < kSmallU; u++) {
+        if (s0 + u * kSmallW >= steps) break;
+        if constexpr (P3) {
+          bf16x8 fb[3], fa[TM][3];
+          auto pieces_of = [&](float(&x)[8], bf16x8(&f)[3]) {
+            uint32_t q[3][4];
+#pragma unroll
+            for (int j = 0; j < 8; j++) x[j] *= kSplitUp;
+            split_run<8>(x, q[0], q[1], q[2], bad);
+#pragma unroll
+            for (int p = 0; p < 3; p++)
+              f[p] = __builtin_bit_cast(bf16x8, uintx4{q[p][0], q[p][1], q[p][2], q[p][3]});
+          };
+          pieces_of(b[u].v, fb);
+#pragma unroll
+          for (int r = 0; r < TM; r++) {
+            pieces_of(a[u][r].v, fa[r]);
+#pragma unroll
+            for (int q = 0; q < 5; q++)
+              lo[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[r][kPieceA[q]], fb[kPieceB[q]], lo[r], 0, 0, 0);
+            acc[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[r][0], fb[0], acc[r], 0, 0, 0);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; j++)
+#pragma unroll
+            for (int r = 0; r < TM; r++)
+              acc[r] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][r].v[j], b[u].v[j], acc[r], 0, 0, 0);
+        }
+      }
+    }
+    if constexpr (P3) {
+#pragma unroll
+      for (int r = 0; r < TM; r++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+          acc[r][v] = (acc[r][v] + lo[r][v]) * kSplitDown;
+          bad |= !(fabsf(acc[r][v]) <= 3.402823466e38f);
+        }
+    }
+  };
+  run(std::integral_constant<bool, PIECES>{});
+  if constexpr (PIECES) {
+    if (__syncthreads_or(bad)) run(std::false_type{});
+  }
+#pragma unroll
+  for (int r = 0; r < TM; r++)
+#pragma unroll
+    for (int v = 0; v < 16; v++)
+      part[w][(r * 32 + 8 * (v >> 2) + 4 * kh + (v & 3)) * 32 + l32] = acc[r][v];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < TM * 2; i++) {
+    const int e = t + 64 * kSmallW * i, row = m0 + e / 32, col = n0 + e % 32;
+    float x = 0.f;
+#pragma unroll
+    for (int q = 0; q < kSmallW; q++) x += part[q][e];
+    if (row < M && col < N) {
+      const int64_t at = (int64_t)blockIdx.y * g.sC + (int64_t)row * g.ldc + col;
+      if (g.mode == kEpiAccum) {
+        g.C[at] += x;
+      } else if (g.mode == kEpiActGrad) {
+        g.C[at] = x * act_deriv(g.aux[(int64_t)row * g.ldaux + col], g.act);
+      } else if (g.C2) {
+        g.C[at] = x;
+        g.C2[at] = act_apply(x, g.act);
+      } else {
+        g.C[at] = act_apply(x, g.act);
+      }
+    }
+  }
+}
+
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // Activation gradients the plain epilogue applies itself: ReLU's (the
@@ -889,6 +1044,29 @@ static Bf3Pick bf3_pick(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t 
   return best;
 }
 
+// Estimated time (us) of gemm_small_kernel: whole rounds of the CUs, each a
+// launch's latency and the wave's share of K (measured: one round of 64 x 32
+// tiles 9 us at K = 512, 15 at 1024, 47 at 4096; of 32 x 32 tiles 30 at 4096).
+static double small_time(const GemmArgs& g, int batch, int cus) {
+  const int tm = g.M > 32 ? 2 : 1;
+  const int64_t wgs = ceil_div(g.M, 32 * tm) * ceil_div(g.N, 32) * batch;
+  return 1. + (double)ceil_div(wgs, cus) * (3. + (tm == 2 ? 0.0105 : 0.0065) * g.K);
+}
+
+// Whether a product runs on gemm_small_kernel: where its estimate is below
+// four fifths of the tiled kernels' best with K split as it may be (their
+// estimate is that much too high where one workgroup sits on a CU).  E.g.
+// 33 x 4096 x 1024: 27 us against 40 with the call; 33 x 4096 x 4096: 57
+// against 52, not taken; 1024 x 512 x 512: 24 against 37; 1024 x 2048 x 512: 52
+// against 43, not taken.
+static bool small_takes(const GemmArgs& g, int batch, int cus) {
+  if (g.groups || g.kseg || g.kitems || g.kchunk || g.a_rows || g.c_rows || g.row_scale || g.mask_out || g.K <= 0)
+    return false;
+  const int64_t most = std::min<int64_t>(32, g.K / 256);
+  const Bf3Pick p = bf3_pick(g.M, g.N, g.K, batch, 0, g.C2 ? 1 : most, cus);
+  return small_time(g, batch, cus) < 0.8 * bf3_time(p.tile, g.M, g.N, g.K, batch, p.splits, cus);
+}
+
 int launch_gemm_ex(const GemmArgs& in, bool tA, bool tB, int batch, hipStream_t s) {
   if (in.M <= 0 || in.N <= 0 || batch <= 0) return 0;
   GemmArgs g = in;
@@ -929,6 +1107,29 @@ int launch_gemm_ex(const GemmArgs& in, bool tA, bool tB, int batch, hipStream_t 
   }
   const int zs = g.kchunk ? (int)ceil_div(g.K, g.kchunk) : 1;
   const int cus = device_cus();
+  // (each operand's own alignment: a row-contiguous one needs none)
+  const bool ka = tA || (aligned16(g.A) && g.lda % 4 == 0 && g.sA % 4 == 0 && g.K % 4 == 0 && g.sAk % 4 == 0);
+  const bool kb = !tB || (aligned16(g.B) && g.ldb % 4 == 0 && g.sB % 4 == 0 && g.K % 4 == 0 && g.sBk % 4 == 0);
+  if (ka && kb && !(tA && tB) && small_takes(g, batch, cus)) {
+    const int tm = g.M > 32 ? 2 : 1;
+    g.tiles_m = (int)ceil_div(g.M, 32 * tm);
+    g.tiles_n = (int)ceil_div(g.N, 32);
+    const dim3 sgrid(g.tiles_m * g.tiles_n, batch), sblock(64 * kSmallW);
+    const bool pieces = !g.f32 && g.K >= kBf3MinK;
+#define NSH_SMALL(TA_, TB_)                                                                              \
+  do {                                                                                                   \
+    if (pieces && tm == 2) hipLaunchKernelGGL((gemm_small_kernel<TA_, TB_, true, 2>), sgrid, sblock, 0, s, g);  \
+    else if (pieces) hipLaunchKernelGGL((gemm_small_kernel<TA_, TB_, true, 1>), sgrid, sblock, 0, s, g);        \
+    else if (tm == 2) hipLaunchKernelGGL((gemm_small_kernel<TA_, TB_, false, 2>), sgrid, sblock, 0, s, g);      \
+    else hipLaunchKernelGGL((gemm_small_kernel<TA_, TB_, false, 1>), sgrid, sblock, 0, s, g);                   \
+  } while (0)
+    if (!tA && !tB) NSH_SMALL(false, false);
+    else if (!tA) NSH_SMALL(false, true);
+    else NSH_SMALL(true, false);
+#undef NSH_SMALL
+    NSH_LAUNCHED();
+    return 0;
+  }
   const bool bf3 = bf3_takes(g, vec, plain, tA, tB);
   int bm = BM, bn = BN, tile = kT128;
   if (bf3 && g.groups) {
@@ -1002,6 +1203,7 @@ static int split_chunk(int K, int splits) { return (int)(ceil_div(ceil_div(K, sp
 
 int gemm_split_count(const GemmArgs& g, int batch) {
   if (!splittable(g) || g.M <= 0 || g.N <= 0 || batch <= 0) return 1;
+  if (small_takes(g, batch, device_cus())) return 1;
   // chunks of at least 256, at most 32 of them; the estimate prices the
   // partial sums against the CUs that a few tiles leave idle
   const int64_t sp =

@@ -100,3 +100,37 @@ def test_operands_of_any_magnitude(scale, variant):
     a, b = A.astype(np.float64), B.astype(np.float64)
     bound = (K + 8) * U * (np.abs(a) @ np.abs(b)) + 2.0 ** -149 * K
     assert np.all(np.abs(got - a @ b) <= bound)
+
+
+# the small kernel: one and two row blocks of 32, edges of its 32 columns,
+# K of one wave's step, of every wave's first step and past the loads in flight
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (1, 10, 256), (31, 33, 16), (33, 31, 20), (64, 64, 132), (65, 97, 516),
+                                   (256, 10, 256), (5, 40, 1100), (70, 32, 2052)])
+@pytest.mark.parametrize("variant", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("act", [0, 6])
+def test_small_product_against_float64(M, N, K, variant, act):
+    print(f"small gemm {variant} M={M} N={N} K={K} act={act}", flush=True)
+    A, B = operands(M, N, K, 5 * M + N + K)
+    got = product(A, B, variant, act=act).astype(np.float64)
+    a, b = A.astype(np.float64), B.astype(np.float64)
+    ref = a @ b
+    # eight partial sums of K / 8 steps each; GELU has a slope of at most 1.13
+    bound = (K + 24) * U * (np.abs(a) @ np.abs(b))
+    if act:
+        from math import erf, sqrt
+        ref = np.vectorize(lambda x: 0.5 * x * (1 + erf(x / sqrt(2))))(ref)
+        bound = 1.13 * bound + 4 * U * np.abs(ref) + 1e-7
+    assert np.all(np.abs(got - ref) <= bound)
+
+
+@pytest.mark.parametrize("variant", ["nn", "nt", "tn"])
+def test_small_product_of_special_values(variant):
+    M, N, K = 40, 36, 136
+    A, B = operands(M, N, K, 4)
+    A[1, 0], A[3, K - 1], A[5, 1], A[7, 2] = np.inf, -np.inf, np.nan, 3.4e38
+    with np.errstate(all="ignore"):
+        ref = oracle.matmul(A.ravel(), B.ravel(), M, K, N).reshape(M, N)
+    got = product(A, B, variant)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+    calm = np.isfinite(ref) & (np.abs(ref) < 1e30)
+    helpers.assert_close(got[calm], ref[calm], f"small gemm beside special values {variant}")
