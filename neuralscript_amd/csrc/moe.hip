@@ -206,6 +206,80 @@ __global__ __launch_bounds__(256) void moe_router_tok_kernel(const float* __rest
   prob[tok] = (sum > 0.f && b >= 0) ? bv / sum : 0.f;
 }
 
+// The logits alone for few tokens: workgroup (x, y) computes 64 tokens x 4 EG
+// experts, wave w experts 4 EG y + EG w .. + EG of all 64 tokens (lane =
+// token), with the sequential-k arithmetic above.  moe_router_tok_kernel would
+// put 1000 tokens on 16 CUs, each wave waiting 1024 times in a row for a
+// scalar load of its weights (183 us of c4's launches); here x and the weights
+// both come through LDS, whose reads are in flight together.
+template <int EG>
+__global__ __launch_bounds__(256) void moe_logits_few_kernel(const float* __restrict__ x, const float* __restrict__ Wg,
+                                                             float* __restrict__ logits, int M, int D, int E) {
+#pragma clang fp contract(off)
+  constexpr int kE = 4 * EG, kWT = kRK * kE / 256;  // experts of the workgroup, weights per thread and slab
+  __shared__ __attribute__((aligned(16))) float xs[2][kRT * kRP];
+  __shared__ __attribute__((aligned(16))) float ws[2][kRK * kE];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int tok0 = blockIdx.x * kRT, e0 = blockIdx.y * kE;
+  float acc[EG];
+#pragma unroll
+  for (int j = 0; j < EG; j++) acc[j] = 0.f;
+  float4 st[2];
+  float wt[kWT];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int f = t + 256 * i, r = f >> 3, k = k0 + (f & 7) * 4;
+      st[i] = (tok0 + r < M && k < D) ? *reinterpret_cast<const float4*>(x + (int64_t)(tok0 + r) * D + k)
+                                      : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int i = 0; i < kWT; i++) {
+      const int f = t + 256 * i, k = k0 + f / kE, e = e0 + f % kE;
+      wt[i] = (k < D && e < E) ? Wg[(int64_t)k * E + e] : 0.f;
+    }
+  };
+  auto store = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int f = t + 256 * i;
+      *reinterpret_cast<float4*>(xs[b] + (f >> 3) * kRP + (f & 7) * 4) = st[i];
+    }
+#pragma unroll
+    for (int i = 0; i < kWT; i++) ws[b][t + 256 * i] = wt[i];
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  for (int k0 = 0, b = 0; k0 < D; k0 += kRK, b ^= 1) {
+    load(k0 + kRK);  // (past the end: zeros, not read)
+    const int kn = min(kRK, D - k0);  // a multiple of 4
+    auto four = [&](int kq) {
+      const float4 xv = *reinterpret_cast<const float4*>(xs[b] + lane * kRP + kq);
+      const float xk[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int j = 0; j < EG; j++) {
+          const float prod = xk[u] * ws[b][(kq + u) * kE + wv * EG + j];
+          acc[j] = acc[j] + prod;
+        }
+    };
+    if (kn == kRK) {
+#pragma unroll
+      for (int kq = 0; kq < kRK; kq += 4) four(kq);
+    } else {
+      for (int kq = 0; kq < kn; kq += 4) four(kq);
+    }
+    store(b ^ 1);
+    __syncthreads();
+  }
+  const int tok = tok0 + lane;
+#pragma unroll
+  for (int j = 0; j < EG; j++)
+    if (tok < M && e0 + wv * EG + j < E) logits[(int64_t)tok * E + e0 + wv * EG + j] = acc[j];
+}
+
 // Router logits for any number of experts: workgroup (token tile, expert
 // tile) computes 64 tokens x 64 experts, each logit a sequential-k fp32 sum
 // with contraction off (the arithmetic of moe_router_kernel), into logits.
@@ -276,6 +350,38 @@ __global__ __launch_bounds__(256) void moe_route_logits_kernel(const float* __re
   }
   best[tok] = b;
   prob[tok] = (sum > 0.f && b >= 0) ? bv / sum : 0.f;
+}
+
+// The same routing with one wave per token (E <= 64, lane = expert): the
+// exponentials side by side, then the sum and the choice over the experts in
+// ascending order, as one thread does them.  For few tokens, where one thread
+// per token would evaluate 64 double exponentials in a row on a handful of CUs.
+__global__ __launch_bounds__(256) void moe_route_wave_kernel(const float* __restrict__ logits,
+                                                             const uint8_t* __restrict__ active,
+                                                             int* __restrict__ best, float* __restrict__ prob, int M,
+                                                             int E) {
+  const int tok = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (tok >= M) return;  // (uniform per wave)
+  const bool live = lane < E && (!active || active[lane]);
+  const float l = lane < E ? logits[(int64_t)tok * E + lane] : 0.f;
+  float mx = live && l > -1.0e30f ? l : -1.0e30f;
+  mx = wave_max(mx);
+  const float v = live ? exp_rn(l - mx) : 0.f;
+  float sum = 0.f, bv = 0.f;
+  int b = -1;
+  for (uint64_t left = __ballot(live); left; left &= left - 1) {
+    const int e = __builtin_ctzll(left);
+    const float x = read_lane(v, e);
+    sum = sum + x;
+    if (b < 0 || x > bv) {
+      b = e;
+      bv = x;
+    }
+  }
+  if (lane == 0) {
+    best[tok] = b;
+    prob[tok] = (sum > 0.f && b >= 0) ? bv / sum : 0.f;
+  }
 }
 
 // In-block rank of each token among same-expert tokens, and block counts.
@@ -502,6 +608,16 @@ int launch_moe_route(const float* x, const float* Wg, const uint8_t* active, con
                        s, x, Wg, w.logits, m, d, e);
     NSH_LAUNCHED();
     hipLaunchKernelGGL(moe_route_logits_kernel, dim3((unsigned)ceil_div(M, 256)), dim3(256), 0, s, w.logits, active,
+                       w.best, w.prob, m, e);
+  } else if (tok_path && w.logits && E > 8 && ceil_div(M, kRT) <= 64) {
+    // up to 4096 tokens: 8 or 16 experts to a workgroup, so that 64 experts
+    // make 4 to 8 workgroups of every 64 tokens
+    const bool two = ceil_div(M, kRT) <= 32;
+    const dim3 g((unsigned)ceil_div(M, kRT), (unsigned)ceil_div(E, two ? 8 : 16));
+    if (two) hipLaunchKernelGGL(moe_logits_few_kernel<2>, g, dim3(256), 0, s, x, Wg, w.logits, m, d, e);
+    else hipLaunchKernelGGL(moe_logits_few_kernel<4>, g, dim3(256), 0, s, x, Wg, w.logits, m, d, e);
+    NSH_LAUNCHED();
+    hipLaunchKernelGGL(moe_route_wave_kernel, dim3((unsigned)ceil_div(M, 4)), dim3(256), 0, s, w.logits, active,
                        w.best, w.prob, m, e);
   } else if (tok_path) {
     const dim3 g((unsigned)ceil_div(M, kRT));
