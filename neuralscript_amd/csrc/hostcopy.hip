@@ -149,10 +149,13 @@ int stage_h2d(HostStage& st, void* dev, const void* host, size_t bytes, hipStrea
   return 0;
 }
 
-int stage_d2h(HostStage& st, void* host, const void* dev, size_t bytes, hipStream_t s) {
+void host_copy(void* dst, const void* src, size_t bytes) { CopyPool::get().copy(dst, src, bytes); }
+
+int stage_d2h(HostStage& st, void* host, const void* dev, size_t bytes, hipStream_t s, void* also) {
   if (bytes < kStageMin) {
     NSH_CHECK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
     NSH_CHECK(hipStreamSynchronize(s));
+    if (also) std::memcpy(also, host, bytes);
     return 0;
   }
   if (stage_init(st, s) != 0) return -1;
@@ -174,6 +177,7 @@ int stage_d2h(HostStage& st, void* host, const void* dev, size_t bytes, hipStrea
     const size_t off = i * kStageChunk, len = std::min(kStageChunk, bytes - off);
     NSH_CHECK(hipEventSynchronize(st.ev[k]));
     CopyPool::get().copy(h + off, st.slot[k], len);
+    if (also) CopyPool::get().copy(static_cast<char*>(also) + off, st.slot[k], len);
     if (i + kStageSlots < n && issue(i + kStageSlots) != 0) return -1;
   }
   return 0;
