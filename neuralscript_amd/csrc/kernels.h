@@ -228,11 +228,11 @@ struct MoeBwdWork {
   int* dirty = nullptr;
 };
 // Ints of MoeBwdWork::kitems and floats of MoeBwdWork::kpart for M tokens:
-// every expert's tokens are cut into chunks (512 tokens, more beyond 16384
-// tokens) for the weight gradients dWe1, dWe2, and the experts with several
-// chunks sum their partials in chunk order afterwards (kpart: at most 64
-// expert gradients).
-size_t moe_bwd_kitem_ints(int64_t M, int64_t E);
+// every expert's tokens are cut into chunks (512 tokens, 128 for small
+// experts, more beyond 16384 or 8192 tokens) for the weight gradients dWe1,
+// dWe2, and the experts with several chunks sum their partials in chunk order
+// afterwards (kpart: at most 64 expert gradients, 128 of small experts).
+size_t moe_bwd_kitem_ints(int64_t M, int64_t D, int64_t H, int64_t E);
 size_t moe_bwd_kpart_floats(int64_t M, int64_t D, int64_t H);
 // Floats of MoeBwdWork::splitk that let dWg = x^T dg (K = M tokens, only
 // D x E outputs) run split over K; 0 when it would not be split.

@@ -703,7 +703,7 @@ int launch_moe_experts(const float* x, const float* We1, const float* We2, const
 //   dH = dpre2 p_b gelu'(u);  dg_e = p_e ((e == b ? dpb : 0) - sd)
 //   dx = dg Wg^T + dH We1[b]^T;  dWg = x^T dg
 //   dWe1[e] = sum over e's tokens of x^T dH;  dWe2[e] = sum of (gelu(u) p_b)^T dout
-// Every product is an fp32-MFMA GEMM: grouped by expert over the sorted rows
+// Every product is a GEMM in gemm.hip: grouped by expert over the sorted rows
 // (dpre2, the expert part of dx), or grouped over each expert's token
 // segment as the contraction (dWe1, dWe2).
 // ============================================================================
@@ -793,16 +793,24 @@ __global__ void fill_zero_kernel(float* __restrict__ p, int64_t n) {
 // 512: 0.29 (one range per expert: 0.49).  The chunk grows with M beyond
 // 16384 tokens so that the partial-sum buffer (its size must cover any
 // routing: 2 * ceil(M / chunk) expert gradients) stays at 64 of them.
-static int64_t kchunk_of(int64_t M) { return std::max<int64_t>(512, ceil_div(ceil_div(M, 32), 16) * 16); }
-static int64_t kitems_max(int64_t M, int64_t E) { return E + ceil_div(M, kchunk_of(M)); }
-static int64_t kreduce_max(int64_t M) { return M / (kchunk_of(M) + 1); }
-static int64_t kslots_max(int64_t M) { return 2 * ceil_div(M, kchunk_of(M)); }
+// Small experts (D H up to 64 K floats: at most four 128 x 128 tiles) take
+// chunks of 128: there the launch is a few workgroups, each a serial chain of
+// K slabs, and the partial sums are small (at most 128 slots, 32 MB).  64 x
+// 256, 8 experts, 4096 tokens: a training step 548 us at 128, 596 at 512,
+// where the product took 43 us; at 1024 x 1024 the figures above hold.
+static int64_t kchunk_of(int64_t M, int64_t D, int64_t H) {
+  const int64_t least = D * H <= 65536 ? 128 : 512;
+  return std::max<int64_t>(least, ceil_div(ceil_div(M, least == 128 ? 64 : 32), 16) * 16);
+}
+static int64_t kitems_max(int64_t M, int64_t D, int64_t H, int64_t E) { return E + ceil_div(M, kchunk_of(M, D, H)); }
+static int64_t kreduce_max(int64_t M, int64_t D, int64_t H) { return M / (kchunk_of(M, D, H) + 1); }
+static int64_t kslots_max(int64_t M, int64_t D, int64_t H) { return 2 * ceil_div(M, kchunk_of(M, D, H)); }
 
-size_t moe_bwd_kitem_ints(int64_t M, int64_t E) {
-  return (size_t)(2 + 4 * kitems_max(M, E) + 3 * kreduce_max(M));
+size_t moe_bwd_kitem_ints(int64_t M, int64_t D, int64_t H, int64_t E) {
+  return (size_t)(2 + 4 * kitems_max(M, D, H, E) + 3 * kreduce_max(M, D, H));
 }
 size_t moe_bwd_kpart_floats(int64_t M, int64_t D, int64_t H) {
-  return kreduce_max(M) > 0 ? (size_t)(kslots_max(M) * D * H) : 0;
+  return kreduce_max(M, D, H) > 0 ? (size_t)(kslots_max(M, D, H) * D * H) : 0;
 }
 
 // kit[0] = items, kit[1] = experts with several chunks; then maxitems items
@@ -993,10 +1001,10 @@ int launch_moe_backward(const float* x, const float* dout, const float* Wg, cons
   NSH_LAUNCHED();
   // token chunks of each expert (without the work buffers: one K range per
   // expert)
-  const bool chunked = b.kitems && (b.kpart || kreduce_max(M) == 0);
-  const int maxitems = (int)kitems_max(M, E), maxred = (int)kreduce_max(M);
+  const bool chunked = b.kitems && (b.kpart || kreduce_max(M, D, H) == 0);
+  const int maxitems = (int)kitems_max(M, D, H, E), maxred = (int)kreduce_max(M, D, H);
   if (chunked) {
-    hipLaunchKernelGGL(moe_kitems_kernel, dim3(1), dim3(256), 0, s, w.seg, (int)E, (int)kchunk_of(M), maxitems,
+    hipLaunchKernelGGL(moe_kitems_kernel, dim3(1), dim3(256), 0, s, w.seg, (int)E, (int)kchunk_of(M, D, H), maxitems,
                        b.kitems, b.dirty);
     NSH_LAUNCHED();
   }
