@@ -7,9 +7,11 @@
 //   reference arithmetic: ns_attention_fwd, codegen.cpp:1724-1777
 //   (per head: s = (q . k) * 1/sqrt(Dk); row softmax; ctx = P V)
 //
-// gfx950 design (wave64, fp32 MFMA 32x32x2):
-//  * Workgroup = 4 waves = 128 queries of one head; each wave owns 32
-//    queries.  Keys/values stream through LDS in 64-key tiles, double
+// gfx950 design (wave64; fp32 products as six bf16 MFMAs 32x32x16 over
+// three-piece operands, split3.h, with the fp32 MFMA 32x32x2 for operands the
+// pieces cannot hold and for dK/dV at head size 128):
+//  * Forward: workgroup = 8 waves = 256 queries of one head; each wave owns 32
+//    queries.  Keys/values stream through LDS in 64-key tiles (pieces), double
 //    buffered with register prefetch.
 //  * Transposed products: S^T = K . Q^T and O^T = V^T . P^T.  In the 32x32
 //    accumulator layout a lane then holds one QUERY column (lane % 32) and 16
@@ -624,8 +626,8 @@ __global__ __launch_bounds__(256) void attn_unpad_kernel(const float* __restrict
 //   dV = P^T dO,  dK = scale dS^T Q,  dQ = scale dS K
 // (ns_attention_bwd, codegen.cpp:1785-1907, computes the same quantities
 // with explicit S x S matrices.)  Two kernels, no atomics:
-//  * dk/dv: one workgroup per 128 keys (32 per wave) loops over query tiles;
-//    it forms S = Q K^T with the KEY as the lane column, so P and dS are the
+//  * dk/dv: one workgroup per 128 keys (32 per pair of waves; 32 per wave in
+//    fp32 MFMA at head size 128) loops over query tiles; it forms S = Q K^T with the KEY as the lane column, so P and dS are the
 //    A operands of dV = P^T dO and dK = dS^T Q directly from registers.
 //  * dq: one workgroup per 128 queries loops over key tiles in the forward's
 //    transposed layout (lane = query): dS^T feeds dQ^T = K^T dS^T.
@@ -1712,8 +1714,16 @@ static int wide_bwd(const float* Q, const float* K, const float* V, const float*
   return 0;
 }
 
+// The tile loads address rows by 32-bit byte offsets inside a 64-row tile:
+// row pitches below 2^24 floats.  Wider arrays go through the padded copies,
+// whose pitch is their own, some heads (2^22 columns) at a time.
+constexpr int64_t kMaxPitch = (int64_t)1 << 24;
+static int64_t heads_at_once(int64_t H, int64_t dkp) {
+  return H * dkp < kMaxPitch ? H : std::max<int64_t>(1, kMaxPitch / 4 / dkp);
+}
+
 bool attention_in_place(int64_t D, int64_t H, int64_t ld, const void* const* ptrs, int n) {
-  if (H <= 0 || D % H != 0 || ld % 4 != 0) return false;
+  if (H <= 0 || D % H != 0 || ld % 4 != 0 || ld >= kMaxPitch) return false;
   const int64_t dk = D / H;
   if (dk != 32 && dk != 64 && dk != 128) return false;
   for (int i = 0; i < n; i++)
@@ -1727,7 +1737,7 @@ size_t attention_pad_floats(int64_t S, int64_t D, int64_t H, bool backward) {
   // wide path: the score block, and in the backward its gradient
   if (!dkp) return (size_t)wide_score_floats(S, H, backward) + wide_split_floats(S, H, D / H);
   // forward: Q K V ctx; backward: Q K V O dO dQ dK dV
-  return (size_t)((backward ? 8 : 4) * S * H * dkp);
+  return (size_t)((backward ? 8 : 4) * S * heads_at_once(H, dkp) * dkp);
 }
 
 static int pad_copy(const float* src, int64_t ld, float* dst, int64_t S, int64_t H, int64_t dk, int64_t dkp,
@@ -1778,16 +1788,21 @@ int launch_attention_fwd(const float* Q, const float* K, const float* V, float* 
     return -1;
   }
   if (!dkp) return wide_fwd(Q, K, V, ctx, lse, S, H, DK, ld, scale, pad_ws, s);
-  const int64_t ldp = H * dkp, n = S * ldp;
+  const int64_t hs = heads_at_once(H, dkp), n = S * hs * dkp;
   float *Qp = pad_ws, *Kp = pad_ws + n, *Vp = pad_ws + 2 * n, *Op = pad_ws + 3 * n;
-  if (pad_copy(Q, ld, Qp, S, H, DK, dkp, s) || pad_copy(K, ld, Kp, S, H, DK, dkp, s) ||
-      pad_copy(V, ld, Vp, S, H, DK, dkp, s))
-    return -1;
-  if (dkp == 128) flash_fwd<128>(Qp, Kp, Vp, Op, lse, S, H, ldp, scale, s);
-  else if (dkp == 64) flash_fwd<64>(Qp, Kp, Vp, Op, lse, S, H, ldp, scale, s);
-  else flash_fwd<32>(Qp, Kp, Vp, Op, lse, S, H, ldp, scale, s);
-  NSH_LAUNCHED();
-  return unpad_copy(Op, ctx, ld, S, H, DK, dkp, s);
+  for (int64_t h = 0; h < H; h += hs) {
+    const int64_t hn = std::min(hs, H - h), ldp = hn * dkp, col = h * DK;
+    float* const l = lse ? lse + h * S : nullptr;
+    if (pad_copy(Q + col, ld, Qp, S, hn, DK, dkp, s) || pad_copy(K + col, ld, Kp, S, hn, DK, dkp, s) ||
+        pad_copy(V + col, ld, Vp, S, hn, DK, dkp, s))
+      return -1;
+    if (dkp == 128) flash_fwd<128>(Qp, Kp, Vp, Op, l, S, hn, ldp, scale, s);
+    else if (dkp == 64) flash_fwd<64>(Qp, Kp, Vp, Op, l, S, hn, ldp, scale, s);
+    else flash_fwd<32>(Qp, Kp, Vp, Op, l, S, hn, ldp, scale, s);
+    NSH_LAUNCHED();
+    if (unpad_copy(Op, ctx + col, ld, S, hn, DK, dkp, s) != 0) return -1;
+  }
+  return 0;
 }
 
 // Row pitch of dS: S rounded up to the dQ pass's key tile.
@@ -1865,17 +1880,21 @@ int launch_attention_bwd(const float* Q, const float* K, const float* V, const f
     return -1;
   }
   if (!dkp) return wide_bwd(Q, K, V, dO, dQ, dK, dV, S, H, DK, ld, scale, pad_ws, s);
-  const int64_t ldp = H * dkp, n = S * ldp;
+  const int64_t hs = heads_at_once(H, dkp), n = S * hs * dkp;
   float* p[8];
   for (int i = 0; i < 8; i++) p[i] = pad_ws + i * n;
   const float* src[5] = {Q, K, V, O, dO};
-  for (int i = 0; i < 5; i++)
-    if (pad_copy(src[i], ld, p[i], S, H, DK, dkp, s) != 0) return -1;
-  if (flash_bwd_any(dkp, p[0], p[1], p[2], p[3], p[4], lse, delta, p[5], p[6], p[7], S, H, ldp, scale, ds, s) != 0)
-    return -1;
   float* dst[3] = {dQ, dK, dV};
-  for (int i = 0; i < 3; i++)
-    if (unpad_copy(p[5 + i], dst[i], ld, S, H, DK, dkp, s) != 0) return -1;
+  for (int64_t h = 0; h < H; h += hs) {
+    const int64_t hn = std::min(hs, H - h), col = h * DK;
+    for (int i = 0; i < 5; i++)
+      if (pad_copy(src[i] + col, ld, p[i], S, hn, DK, dkp, s) != 0) return -1;
+    if (flash_bwd_any(dkp, p[0], p[1], p[2], p[3], p[4], lse + h * S, delta + h * S, p[5], p[6], p[7], S, hn, hn * dkp,
+                      scale, ds, s) != 0)
+      return -1;
+    for (int i = 0; i < 3; i++)
+      if (unpad_copy(p[5 + i], dst[i] + col, ld, S, hn, DK, dkp, s) != 0) return -1;
+  }
   return 0;
 }
 

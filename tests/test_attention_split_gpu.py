@@ -168,3 +168,34 @@ def test_gradients_of_values_without_three_pieces(dk):
             assert np.max(np.abs(g[:, other] - c[:, other])) <= bar(S, c[:, other])
             assert not np.any(np.isfinite(g[:, :dk][~np.isfinite(r[:, :dk])]) &
                               (np.abs(g[:, :dk][~np.isfinite(r[:, :dk])]) < 1e30))
+
+
+def test_rows_too_wide_for_the_tile_offsets():
+    """Rows of 2^24 floats and more: a tile's 32-bit offsets cannot reach its
+    last row, so the heads run in groups on copies.  The columns repeat 1024
+    heads 528 times; every repetition equals those 1024 heads alone."""
+    S, dk, H, reps = 64, 32, 1024, 528
+    D = H * dk
+    assert (S - 1) * D * reps * 4 >= 2 ** 32
+    print(f"attention of {reps * H} heads", flush=True)
+
+    def run(Q, K, V, dO, heads, want=None):
+        n = Q.shape[1]
+        q, k, v, do = (DA.from_host(a) for a in (Q, K, V, dO))
+        ctx, lse = DA(S * n), DA(S * heads)
+        runtime.op("attention_fwd", q, k, v, ctx, lse, S, n, heads)
+        grads = [DA(S * n) for _ in range(3)]
+        ws = DA(runtime.lib().nsh_op_attention_bwd_workspace(S, n, heads, 1) // 4)
+        runtime.op("attention_bwd", q, k, v, ctx, do, lse, *grads, S, n, heads, 1, ws)
+        out = []
+        for i, a in enumerate([ctx, *grads]):
+            a = a.to_host().reshape(S, n)
+            out.append(a if want is None else
+                       all(np.array_equal(a[:, j:j + D], want[i]) for j in range(0, n, D)))
+        for a in (q, k, v, do, ctx, lse, ws, *grads):
+            a.free()
+        return out
+
+    base = inputs(S, D, 77, 4)
+    want = run(*base, H)
+    assert all(run(*(np.tile(a, (1, reps)) for a in base), reps * H, want))
