@@ -146,7 +146,8 @@ int nsh_profile_report(ns_model* m, char* buf, size_t len);
  * A[m*lda+k]; opB(B)[k,n] = transB ? B[n*ldb+k] : B[k*ldb+n].
  * Replaces ns_matmul + ns_act2 (codegen.cpp:1257-1265, 1244-1255),
  * ns_matmul_grad_a (transB, :1318-1326) and ns_matmul_grad_w (transA,
- * :1329-1337); fp32 MFMA. */
+ * :1329-1337); fp32 products (exact operands, fp32 sums) on the matrix
+ * cores. */
 int nsh_op_gemm(const float* A, const float* B, float* C, int64_t M, int64_t N, int64_t K,
                 int64_t lda, int64_t ldb, int64_t ldc, int transA, int transB, int act);
 

@@ -1,4 +1,4 @@
-// fp32 MFMA GEMM for gfx950 (CDNA4):  C[M,N] = act( opA(A) . opB(B) ).
+// fp32 GEMM for gfx950 (CDNA4):  C[M,N] = act( opA(A) . opB(B) ).
 //
 // Replaces the reference's dense products and their activation passes:
 //   ns_matmul + ns_act2          /root/reference/src/codegen/codegen.cpp:1257-1265, 1244-1255

@@ -13,13 +13,15 @@
 //    this kernel), and exp is evaluated in double precision and rounded once
 //    to float, i.e. correctly rounded, which glibc's expf also is except
 //    within ~0.002 ulp of a rounding boundary.  x and Wg slabs are staged in
-//    LDS; each thread owns 16 tokens x E/64 experts.
+//    LDS; each thread owns 16 tokens x E/64 experts.  Up to 4096 tokens that
+//    is too few workgroups, each a serial chain over k: the experts are dealt
+//    over workgroups too (moe_logits_few_kernel).
 //  * Dispatch: per 256-token block, each token's rank among the block's
 //    tokens of the same expert and the block's per-expert counts; one scan
 //    turns those into expert segments and a STABLE permutation (tokens stay
 //    in order within their expert), plus the (expert, m-tile) list of the
 //    grouped GEMM -- all on the device, no host round trip.
-//  * Experts: two grouped fp32-MFMA GEMMs over the expert-sorted rows: the
+//  * Experts: two grouped GEMMs (gemm.hip) over the expert-sorted rows: the
 //    first gathers x rows through the permutation and applies GELU in its
 //    epilogue, the second scatters rows back to token order scaled by p.
 #include <type_traits>
@@ -211,7 +213,8 @@ __global__ __launch_bounds__(256) void moe_router_tok_kernel(const float* __rest
 // token), with the sequential-k arithmetic above.  moe_router_tok_kernel would
 // put 1000 tokens on 16 CUs, each wave waiting 1024 times in a row for a
 // scalar load of its weights (183 us of c4's launches); here x and the weights
-// both come through LDS, whose reads are in flight together.
+// both come through LDS, whose reads are in flight together (the whole call on
+// 1000 tokens: 167 -> 108 us).
 template <int EG>
 __global__ __launch_bounds__(256) void moe_logits_few_kernel(const float* __restrict__ x, const float* __restrict__ Wg,
                                                              float* __restrict__ logits, int M, int D, int E) {
