@@ -108,8 +108,8 @@ int launch_embedding_grad(const float* dout, const float* idx, float* dW, int64_
 // ctx[S, D] (heads concatenated) = softmax(Q_h K_h^T * scale) V_h per head,
 // Q/K/V row-major [S, D] with row pitch ld.  lse (optional, [H, S]) receives
 // log2(sum_j 2^(s_j * scale * log2 e)) per query, for the backward pass.
-// Head sizes 32, 64 and 128 on 16-byte aligned rows (ld % 4 == 0) run in
-// place (attention_in_place over the arrays read as float4 rows: Q, K, V,
+// Head sizes 32, 64 and 128 on 16-byte aligned rows (ld % 4 == 0, below 2^24
+// floats) run in place (attention_in_place over the arrays read as float4 rows: Q, K, V,
 // and O, dO in the backward); every other head size up to 128 runs on a copy
 // padded with zero columns to the next of them, in pad_ws
 // (attention_pad_floats floats).  Above 128, pad_ws (as many floats) holds
