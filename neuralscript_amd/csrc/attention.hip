@@ -9,7 +9,11 @@
 //
 // gfx950 design (wave64; fp32 products as six bf16 MFMAs 32x32x16 over
 // three-piece operands, split3.h, with the fp32 MFMA 32x32x2 for operands the
-// pieces cannot hold and for dK/dV at head size 128):
+// pieces cannot hold and for dK/dV at head size 128).  An infinity, a NaN or an
+// overflow shows only at the end of a workgroup's loop, which then runs a
+// second time in fp32, without prefetch: one such key in every head costs 610
+// us forward and 2190 backward where 250 and 780 are the rule (3001 tokens, 16
+// heads of 64; fp32 MFMA alone took 410 and 1360).
 //  * Forward: workgroup = 8 waves = 256 queries of one head; each wave owns 32
 //    queries.  Keys/values stream through LDS in 64-key tiles (pieces), double
 //    buffered with register prefetch.
@@ -246,6 +250,8 @@ __device__ __forceinline__ void flash_fwd_f32(const float* __restrict__ Q, const
 // One K tile (KT keys x DK) split into pieces on its way to LDS, as the A
 // operand of S^T = K Q^T: [piece][dim / 8][key] chunks of 8 bf16.  NTH
 // threads starting at t = 0, one chunk (8 dims of a key, two float4) each.
+// Rows past the end are copies of the last row, here and in VPieces: their
+// probabilities are zeros (a masked key's score, or a query's lse = +inf).
 template <int DK, int KT>
 struct KPieces {
   static constexpr int kItems = KT * DK / 8;
@@ -253,10 +259,8 @@ struct KPieces {
   static constexpr int kPiece = DK / 8 * kChunk;
   static constexpr int kBytes = 3 * kPiece;
   float v[8];
-  bool in = false;  // the key exists
   __device__ __forceinline__ void load(const float* __restrict__ X, int64_t ld, int hcol, int key0, int S, int t) {
     const int key = t / (DK / 8), c = t % (DK / 8);
-    in = key0 + key < S;
     // wave-uniform tile address + 32-bit offset inside the tile
     const char* base = reinterpret_cast<const char*>(X + (int64_t)key0 * ld + hcol);
     const uint32_t off = ((uint32_t)min(key, S - 1 - key0) * (uint32_t)ld + c * 8) * 4u;
@@ -268,7 +272,7 @@ struct KPieces {
     const int key = t / (DK / 8), c = t % (DK / 8);
     uint32_t w[3][4];
 #pragma unroll
-    for (int j = 0; j < 8; j++) v[j] = in ? v[j] : 0.f;
+    for (int j = 0; j < 8; j++) v[j] *= kSplitUp;
     split_run<8>(v, w[0], w[1], w[2], bad);
 #pragma unroll
     for (int p = 0; p < 3; p++)
@@ -292,13 +296,11 @@ struct VPieces {
   static constexpr int kPiece = KT / 8 * DK * 16;
   static constexpr int kBytes = 3 * kPiece;
   float v[8];
-  int lim = 0;  // tile rows below lim exist
   __device__ __forceinline__ static int row_of(int c, int j) {
     return PERM ? (c >> 2) * 32 + ((c >> 1) & 1) * 16 + (c & 1) * 4 + (j & 3) + 8 * (j >> 2) : c * 8 + j;
   }
   __device__ __forceinline__ void load(const float* __restrict__ X, int64_t ld, int hcol, int row0, int S, int t) {
-    const int c = t / DK, d = t % DK;
-    lim = S - row0;
+    const int c = t / DK, d = t % DK, lim = S - row0;  // tile rows below lim exist
     const char* base = reinterpret_cast<const char*>(X + (int64_t)row0 * ld + hcol);
 #pragma unroll
     for (int j = 0; j < 8; j++)
@@ -308,7 +310,7 @@ struct VPieces {
     const int c = t / DK, d = t % DK;
     uint32_t w[3][4];
 #pragma unroll
-    for (int j = 0; j < 8; j++) v[j] = row_of(c, j) < lim ? v[j] : 0.f;
+    for (int j = 0; j < 8; j++) v[j] *= kSplitUp;
     split_run<8>(v, w[0], w[1], w[2], bad);
 #pragma unroll
     for (int p = 0; p < 3; p++)
@@ -320,13 +322,15 @@ struct VPieces {
   }
 };
 
-// 8 fp32 values as the three operand pieces of an MFMA step.
+// 8 fp32 values (probabilities, dS), times kSplitUp, as the three operand
+// pieces of an MFMA step.  Not checked: what they cannot hold leaves a sum that
+// is not finite, which is.
 __device__ __forceinline__ void split8(const float* v, bf16x8 (&f)[3]) {
   uintx4 w[3];
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     uint32_t a, b, c;
-    split_pair(v[2 * j], v[2 * j + 1], a, b, c);
+    split_pair(v[2 * j] * kSplitUp, v[2 * j + 1] * kSplitUp, a, b, c);
     w[0][j] = a; w[1][j] = b; w[2][j] = c;
   }
 #pragma unroll
@@ -340,8 +344,8 @@ constexpr int fwd_keys() {
   return DK == 128 ? 32 : 64;
 }
 
-// S^T tile (KT keys x this wave's 32 queries) = K_tile Q^T, in log2 units
-// (Q is pre-scaled by scale * log2(e)).
+// Raw scores (KT keys x this wave's 32 queries) = K_tile Q^T of the scaled
+// pieces: kSplitUp^2 = 1 / kSplitDown times the product.
 template <int DK, int KT>
 __device__ __forceinline__ void score_pieces(const char* __restrict__ ks, const bf16x8 (&qf)[DK / 16][3], int l32,
                                              int kh, floatx16 (&sc)[KT / 32]) {
@@ -412,7 +416,8 @@ __global__ __launch_bounds__(kFW * 64, 2) void flash_fwd_kernel(const float* __r
   float m = -INFINITY, l = 0.f;
   bool bad = false;
   {
-    // B operand of S^T = K Q^T: this lane's query (pre-scaled), head dims 16 g + 8 kh + (0..7).
+    // B operand of S^T = K Q^T: this lane's query (times scale * log2(e), so that
+    // scores are in log2 units), head dims 16 g + 8 kh + (0..7).
     bf16x8 qf[DK / 16][3];
 #pragma unroll
     for (int g = 0; g < DK / 16; g++) {
@@ -422,7 +427,7 @@ __global__ __launch_bounds__(kFW * 64, 2) void flash_fwd_kernel(const float* __r
       float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
       uint32_t u[3][4];
 #pragma unroll
-      for (int j = 0; j < 8; j++) x[j] *= scale_log2;
+      for (int j = 0; j < 8; j++) x[j] *= scale_log2 * kSplitUp;
       split_run<8>(x, u[0], u[1], u[2], bad);
 #pragma unroll
       for (int p2 = 0; p2 < 3; p2++)
@@ -483,7 +488,7 @@ __global__ __launch_bounds__(kFW * 64, 2) void flash_fwd_kernel(const float* __r
 #pragma unroll
         for (int v = 0; v < 16; v++) mloc = fmaxf(mloc, sc[kb][v]);
       mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
-      const float mnew = fmaxf(m, mloc);
+      const float mnew = fmaxf(m, mloc * kSplitDown);
       if (__any(mnew > m)) {
         const float corr = exp2_hw(m - mnew);
         l *= corr;
@@ -497,7 +502,7 @@ __global__ __launch_bounds__(kFW * 64, 2) void flash_fwd_kernel(const float* __r
       for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
         for (int v = 0; v < 16; v++) {
-          const float p = exp2_hw(sc[kb][v] - mnew);
+          const float p = exp2_hw(fmaf(sc[kb][v], kSplitDown, -mnew));
           sc[kb][v] = p;
           lsum += p;
         }
@@ -568,14 +573,15 @@ __global__ __launch_bounds__(kFW * 64, 2) void flash_fwd_kernel(const float* __r
 #pragma unroll
     for (int v = 0; v < 16; v++) bad |= !(fabsf(o[d][v]) <= 3.402823466e38f);
   float* const sm = reinterpret_cast<float*>(smem);
-  if (__syncthreads_or(bad)) flash_fwd_f32<DK>(Q, K, V, sm, S, ld, hcol, q0, scale_log2, o, m, l);
+  const bool f32 = __syncthreads_or(bad);
+  if (f32) flash_fwd_f32<DK>(Q, K, V, sm, S, ld, hcol, q0, scale_log2, o, m, l);
 
   // Row statistics for the backward pass: log2-sum-exp of the scaled scores.
   if (lse && kh == 0 && qrow < S) lse[(int64_t)h * S + qrow] = m + log2f(l);
 
   // O^T (d, query) / l  ->  LDS [query][d]  ->  coalesced rows of ctx.
   static_assert(kFW * 32 * (DK + 1) * 4 <= (int)sizeof(smem), "output staging fits the K/V buffers");
-  const float inv = 1.f / l;
+  const float inv = (f32 ? 1.f : kSplitDown) / l;
   float* T = sm + w * 32 * (DK + 1);
 #pragma unroll
   for (int d = 0; d < NDB; d++)
@@ -708,17 +714,18 @@ __device__ __forceinline__ void put_block(float* __restrict__ buf, int lane, con
   for (int g = 0; g < 4; g++)
     *reinterpret_cast<float4*>(buf + (g * 64 + lane) * 4) = make_float4(x[4 * g], x[4 * g + 1], x[4 * g + 2], x[4 * g + 3]);
 }
-// x = P o (x - delta), P from put_block, delta of the block's 32 queries.
+// x = P o (f x - delta), P from put_block, delta of the block's 32 queries; f =
+// 1, or kSplitDown for a product of pieces.
 __device__ __forceinline__ void take_ds(const float* __restrict__ buf, const float* __restrict__ delta, int lane,
-                                        int kh, floatx16& x) {
+                                        int kh, float f, floatx16& x) {
 #pragma unroll
   for (int g = 0; g < 4; g++) {
     const float4 p = *reinterpret_cast<const float4*>(buf + (g * 64 + lane) * 4);
     const float4 d = *reinterpret_cast<const float4*>(delta + 8 * g + 4 * kh);
-    x[4 * g] = p.x * (x[4 * g] - d.x);
-    x[4 * g + 1] = p.y * (x[4 * g + 1] - d.y);
-    x[4 * g + 2] = p.z * (x[4 * g + 2] - d.z);
-    x[4 * g + 3] = p.w * (x[4 * g + 3] - d.w);
+    x[4 * g] = p.x * fmaf(x[4 * g], f, -d.x);
+    x[4 * g + 1] = p.y * fmaf(x[4 * g + 1], f, -d.y);
+    x[4 * g + 2] = p.z * fmaf(x[4 * g + 2], f, -d.z);
+    x[4 * g + 3] = p.w * fmaf(x[4 * g + 3], f, -d.w);
   }
 }
 // x = P = 2^(c x - lse); keys past the end: exponent -inf (kneg), P = 0; lse
@@ -785,7 +792,7 @@ __device__ __forceinline__ void flash_bwd_dkdv_f32(const float* __restrict__ Q, 
       }
       __syncthreads();
       if (role) {
-        take_ds(pbuf, ls + 64 + qb * 32, lane, kh, x);
+        take_ds(pbuf, ls + 64 + qb * 32, lane, kh, 1.f, x);
         if constexpr (STORE_DS) store_ds_rows(x, dS, (int64_t)h * S, it * 64 + qb * 32, key, kh, S, ldds);
       }
       // step s pairs query 8(s/4) + 4kh + s%4
@@ -922,8 +929,10 @@ __global__ __launch_bounds__(kPNT, 2) void flash_bwd_dkdv_kernel(
       const float* p = X + (int64_t)(key < S ? key : S - 1) * ld + hcol + 16 * g + 8 * kh;
       const float4 a = keep4(key < S, *reinterpret_cast<const float4*>(p));
       const float4 b = keep4(key < S, *reinterpret_cast<const float4*>(p + 4));
-      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
       uint32_t u[3][4];
+#pragma unroll
+      for (int j = 0; j < 8; j++) x[j] *= kSplitUp;
       split_run<8>(x, u[0], u[1], u[2], bad);
 #pragma unroll
       for (int q = 0; q < 3; q++) xf[g][q] = __builtin_bit_cast(bf16x8, uintx4{u[q][0], u[q][1], u[q][2], u[q][3]});
@@ -949,10 +958,10 @@ __global__ __launch_bounds__(kPNT, 2) void flash_bwd_dkdv_kernel(
         __builtin_amdgcn_s_setprio(0);
         const float* st = reinterpret_cast<const float*>(cur + Tile::kStat);
         if (!role) {
-          take_p(st, kh, c_log2, kneg, x[0]);
+          take_p(st, kh, c_log2 * kSplitDown, kneg, x[0]);
           put_block(pbuf + (it & 1) * 1024, lane, x[0]);
         } else {
-          take_ds(pbuf + (it & 1) * 1024, st, lane, kh, x[0]);
+          take_ds(pbuf + (it & 1) * 1024, st, lane, kh, kSplitDown, x[0]);
           if constexpr (STORE_DS) store_ds_rows(x[0], dS, hS, it * 32, key, kh, S, ldds);
         }
         // the next tile, here so that its registers are not held over the products
@@ -968,12 +977,13 @@ __global__ __launch_bounds__(kPNT, 2) void flash_bwd_dkdv_kernel(
   for (int d = 0; d < NDB; d++)
 #pragma unroll
     for (int v = 0; v < 16; v++) bad |= !(fabsf(acc[d][v]) <= 3.402823466e38f);
-  if (__syncthreads_or(bad))
+  const bool f32 = __syncthreads_or(bad);
+  if (f32)
     flash_bwd_dkdv_f32<DK, STORE_DS>(Q, X, dO, lse, delta, dS, reinterpret_cast<float*>(smem), S, h, key, role, ld,
                                      c_log2, ldds, acc);
   // accumulator v of block d: key 8(v/4) + 4kh + v%4 of the pair's, head dim d*32 + l32
   float* __restrict__ out = role ? dK : dV;
-  const float f = role ? scale : 1.f;
+  const float f = (role ? scale : 1.f) * (f32 ? 1.f : kSplitDown);
 #pragma unroll
   for (int d = 0; d < NDB; d++)
 #pragma unroll
@@ -1313,7 +1323,8 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_ds_kernel(const float* __
   for (int d = 0; d < NDB; d++)
 #pragma unroll
     for (int v = 0; v < 16; v++) bad |= !(fabsf(acc[d][v]) <= 3.402823466e38f);
-  if (__syncthreads_or(bad)) {
+  const bool f32 = __syncthreads_or(bad);
+  if (f32) {
     // K values the split cannot hold, or a dS that is not finite: fp32 MFMA
     constexpr int P = DK + 4;
     float* ks = reinterpret_cast<float*>(smem);
@@ -1345,10 +1356,11 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_ds_kernel(const float* __
   // dQ^T (d, query) -> LDS [query][d] -> rows of dQ
   __syncthreads();  // the tiles are read; T takes their place
   float* T = reinterpret_cast<float*>(smem) + w * 32 * (DK + 1);
+  const float f = f32 ? scale : scale * kSplitDown;
 #pragma unroll
   for (int d = 0; d < NDB; d++)
 #pragma unroll
-    for (int v = 0; v < 16; v++) T[l32 * (DK + 1) + d * 32 + 8 * (v >> 2) + 4 * kh + (v & 3)] = acc[d][v] * scale;
+    for (int v = 0; v < 16; v++) T[l32 * (DK + 1) + d * 32 + 8 * (v >> 2) + 4 * kh + (v & 3)] = acc[d][v] * f;
   __syncthreads();
   for (int r = 0; r < 32; r++) {
     const int q = q0 + w * 32 + r;

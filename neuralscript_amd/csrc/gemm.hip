@@ -555,13 +555,6 @@ __global__ __launch_bounds__(NT, VEC ? 4 : 1) void gemm_f32_kernel(GemmArgs g) {
 
 // ---- three-piece bf16 kernel ---------------------------------------------------
 
-// Operands are scaled by 2^24 before they are split, and the accumulators by
-// 2^-48 after the K loop (all exact): the last piece then stays above bf16's
-// smallest subnormal for every fp32 operand down to 2^-134, so a gradient's
-// softmax tails do not take the fp32 path.  The scaled sums overflow where a
-// result exceeds 2^80; such tiles take the fp32 path too.
-constexpr float kSplitUp = 0x1p24f, kSplitDown = 0x1p-48f;
-
 // LDS layout of one operand's 16-wide K slab: [piece][k / 8][row] chunks of 8
 // bf16.  The two k-halves are 64 bytes further apart than ROWS chunks, so the
 // staging stores of a k-contiguous operand (8 lanes = 4 rows x 2 halves)

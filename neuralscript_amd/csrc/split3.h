@@ -16,11 +16,14 @@
 // 3.4e-7, 4096 1.2e-6 -> 1.0e-6, 16384 2.3e-6 -> 2.1e-6; uniform [0, 1)
 // operands 6.2e-8 -> 3.2e-8, ..., 1.7e-6 -> 1.1e-6.
 //
-// What the split cannot hold is flagged and computed by fp32 MFMA instead:
-// infinities, NaN and values that round to infinity in bf16 (their remainder
-// is NaN), and values so small that the last piece would fall below bf16's
-// smallest subnormal, 2^-133 (their remainder is an fp32 subnormal; values
-// of at least 2^-102 never are).  bf16 MFMA keeps subnormal operands.
+// Operands are scaled by kSplitUp = 2^24 before they are split, and the sums by
+// kSplitDown = 2^-48 (all exact): the last piece then stays above bf16's
+// smallest subnormal, 2^-133, for every fp32 operand down to 2^-134, so a
+// gradient's or a softmax's tails keep their bits.  bf16 MFMA keeps subnormal
+// operands.  What the split cannot hold is flagged and computed by fp32 MFMA
+// instead: infinities, NaN and operands past 2^103 (their remainder is NaN),
+// operands below 2^-134 (their remainder is an fp32 subnormal), and sums past
+// 2^80, which overflow.
 #pragma once
 #include "common.h"
 
@@ -40,6 +43,8 @@ __device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
 }
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
+
+constexpr float kSplitUp = 0x1p24f, kSplitDown = 0x1p-48f;
 
 // signaling / quiet NaN, -inf, +inf, -subnormal, +subnormal
 constexpr int kUnsplittable = 0x1 | 0x2 | 0x4 | 0x200 | 0x10 | 0x80;

@@ -170,6 +170,53 @@ def test_gradients_of_values_without_three_pieces(dk):
                               (np.abs(g[:, :dk][~np.isfinite(r[:, :dk])]) < 1e30))
 
 
+def error_norms(got, refs):
+    return [np.linalg.norm(g.astype(np.float64) - r) for g, r in zip(got, refs)]
+
+
+# from full-size gradients down to where the operand itself is subnormal
+@pytest.mark.parametrize("exponent", [-90, -100, -108, -115, -126])
+@pytest.mark.parametrize("dk", [32, 64, 128])
+@pytest.mark.parametrize("store_ds", [0, 1])
+@pytest.mark.parametrize("which", [2, 3])
+def test_gradients_of_any_magnitude(exponent, dk, store_ds, which):
+    """V or dO times a power of two, which is exact: the gradients it enters
+    scale with it and their errors may only scale with them (a quarter is left
+    to the other rounding of the fp32 loop, which one subnormal operand sends a
+    workgroup to), besides what fp32 has no bits for: 2^-149 a product, over S
+    products and the row of dS that each comes from."""
+    print(f"attention gradients dk={dk} store_ds={store_ds} operand {which} * 2^{exponent}", flush=True)
+    S, H = 200, 2
+    arrs = inputs(S, H * dk, 41, 4)
+    base = error_norms(gradients(*arrs, H, store_ds), reference_gradients(*arrs, H))
+    f = 2.0 ** exponent
+    arrs[which] = (arrs[which] * np.float32(f)).astype(np.float32)
+    refs = reference_gradients(*arrs, H)
+    errs = error_norms(gradients(*arrs, H, store_ds), refs)
+    least = 2.0 ** -149 * 4 * S * np.sqrt(S * H * dk)
+    for name, e, b, unscaled in zip(("dQ", "dK", "dV"), errs, base, (False, False, which == 2)):
+        assert e <= 1.25 * b * (1.0 if unscaled else f) + least, name
+
+
+@pytest.mark.parametrize("dk", [32, 64, 128])
+def test_output_of_a_lone_small_probability(dk):
+    """Only one key has a value, and its score lies 85 to 86 below the others':
+    the output is that value times a probability of about 2^-123, of which
+    unscaled bf16 pieces would keep 11 bits."""
+    S, H = 130, 1
+    rng = np.random.default_rng(dk)
+    Q, K, V = (np.zeros((S, dk), np.float32) for _ in range(3))
+    Q[:, 0] = np.sqrt(np.float32(dk)) * (8.5 + 0.1 * rng.random(S)).astype(np.float32)
+    K[77, 0] = -10.0
+    V[77] = 2.0 ** 30 * (1 + rng.random(dk)).astype(np.float32)
+    got, _ = core(Q, K, V, H)
+    ref = reference(Q, K, V, H)
+    # the exponential's argument, 123 in log2 units, is rounded three times
+    # (query, score, difference) to 2^-24 of itself; the sums as bar()
+    bound = 3 * 124 * np.log(2) * 2.0 ** -24 + 2.0 ** -24 * (16 + 2 * np.sqrt(S))
+    assert np.max(np.abs(got / ref - 1)) <= bound
+
+
 def test_rows_too_wide_for_the_tile_offsets():
     """Rows of 2^24 floats and more: a tile's 32-bit offsets cannot reach its
     last row, so the heads run in groups on copies.  The columns repeat 1024
