@@ -1616,7 +1616,7 @@ static size_t wide_split_floats(int64_t S, int64_t H, int64_t dk) {
   for (const int64_t nq : {rows, S % rows})
     if (nq > 0) {
       const GemmArgs g = wide_pv_args(nq, S, dk);
-      m = std::max(m, gemm_split_workspace(g, (int)H, gemm_split_count(g, (int)H)));
+      m = std::max(m, gemm_split_workspace(g, (int)H, gemm_split_most(g, (int)H)));
     }
   return m;
 }
@@ -1671,7 +1671,8 @@ static int wide_fwd(const float* Q, const float* K, const float* V, float* ctx, 
     g.A = ws; g.lda = S; g.sA = nq * S;
     g.B = V; g.ldb = ld; g.sB = dk;
     g.C = ctx + q0 * ld; g.ldc = ld; g.sC = dk;
-    if (launch_gemm_split(g, false, false, (int)H, gemm_split_count(g, (int)H), ws + wide_score_floats(S, H, false), s))
+    const int sp = gemm_split_count(g, false, false, (int)H);
+    if (launch_gemm_split(g, false, false, (int)H, sp, ws + wide_score_floats(S, H, false), s))
       return -1;
   }
   return 0;
@@ -1720,7 +1721,8 @@ static int wide_bwd(const float* Q, const float* K, const float* V, const float*
     q.A = G; q.lda = S; q.sA = nq * S;
     q.B = K; q.ldb = ld; q.sB = dk;
     q.C = dQ + q0 * ld; q.ldc = ld; q.sC = dk;
-    if (launch_gemm_split(q, false, false, (int)H, gemm_split_count(q, (int)H), ws + wide_score_floats(S, H, true), s))
+    const int sp = gemm_split_count(q, false, false, (int)H);
+    if (launch_gemm_split(q, false, false, (int)H, sp, ws + wide_score_floats(S, H, true), s))
       return -1;
   }
   return 0;

@@ -963,6 +963,25 @@ __global__ __launch_bounds__(64 * kSmallW, 2) void gemm_small_kernel(GemmArgs g)
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// Whether both operands can be read as float4: each one's contiguous extent,
+// leading dimension, batch stride and base 4-float aligned.  (K-grouped
+// segments start anywhere, so a k-contiguous operand needs the scalar path
+// there.)
+static bool reads_float4(const GemmArgs& g, bool tA, bool tB) {
+  const bool seg = g.kseg || g.kitems;
+  const bool va = aligned16(g.A) && g.lda % 4 == 0 && g.sA % 4 == 0 && ((tA ? g.M : g.K) % 4 == 0) && (tA || !seg);
+  const bool vb = aligned16(g.B) && g.ldb % 4 == 0 && g.sB % 4 == 0 && ((tB ? g.K : g.N) % 4 == 0) && (!tB || !seg);
+  return va && vb && (!g.kblk || (g.sAk % 4 == 0 && g.sBk % 4 == 0));
+}
+
+// Whether gemm_small_kernel can read the operands: a row-contiguous one at any
+// alignment, a k-contiguous one as float4; not both transposed.
+static bool small_reads(const GemmArgs& g, bool tA, bool tB) {
+  const bool ka = tA || (aligned16(g.A) && g.lda % 4 == 0 && g.sA % 4 == 0 && g.K % 4 == 0 && g.sAk % 4 == 0);
+  const bool kb = !tB || (aligned16(g.B) && g.ldb % 4 == 0 && g.sB % 4 == 0 && g.K % 4 == 0 && g.sBk % 4 == 0);
+  return ka && kb && !(tA && tB);
+}
+
 // Activation gradients the plain epilogue applies itself: ReLU's (the
 // training MLPs'); the others take the general epilogue.
 static bool plain_act_grad(const GemmArgs& g) { return g.mode == kEpiActGrad && g.aux && g.act == kActRelu; }
@@ -1000,42 +1019,45 @@ static bool bf3_takes(const GemmArgs& g, bool vec, bool plain, bool tA, bool tB)
 // ---- which kernel, which tile, how many K chunks --------------------------------
 
 // The split kernel's tiles, by use: 256x128 (8 waves, one workgroup on a CU),
-// 128x128 (4 waves, two on a CU), and for grouped products 128x256.
-enum Bf3Tile : int { kT256x128 = 0, kT128, kTiles };
+// 128x128 (4 waves, two on a CU), and for grouped products 128x256; and the
+// fp32 kernel's one, 128x128.
+enum Tile : int { kT256x128 = 0, kT128, kBf3Tiles, kTF32 = kBf3Tiles };
 
 // Estimated time (us) of M x N x K (x batch) on one tile shape with the K
 // range cut into `splits`: whole rounds of the CUs, each tile with a prologue
 // and epilogue worth ~64 steps of K.  Measured rates (N(0,1) operands): 256x128
 // tiles 210 TFLOP/s, 128x128 190 with two workgroups on a CU and ~130 with
-// one.  The splits' partial sums are written and read once more at ~4 TB/s.
-static double bf3_time(int tile, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t splits, int cus) {
-  const int64_t bm = tile == kT128 ? 128 : 256, bn = 128;
+// one; the fp32 kernel two thirds of that.  The splits' partial sums are
+// written and read once more at ~4 TB/s.
+static double tile_time(int tile, int64_t M, int64_t N, int64_t K, int64_t batch, int64_t splits, int cus) {
+  const int64_t bm = tile == kT256x128 ? 256 : 128, bn = 128;
   const int64_t tiles = ceil_div(M, bm) * ceil_div(N, bn) * batch * splits;
   const int64_t n = ceil_div(tiles, cus);  // tiles of the busiest CU
-  const double rate = (tile == kT256x128 ? 210. : n >= 2 ? 190. : 130.) * 1e6 / cus;  // FLOP per us and CU
+  const double bf3 = tile == kT256x128 ? 210. : n >= 2 ? 190. : 130.;
+  const double rate = (tile == kTF32 ? bf3 * 2 / 3 : bf3) * 1e6 / cus;  // FLOP per us and CU
   const double t = (double)n * 2. * bm * bn * ((double)ceil_div(K, splits) + 64.) / rate;
   return splits > 1 ? t + 6. + (double)M * N * batch * splits * 8. / 4e6 : t;
 }
 
-struct Bf3Pick {
+struct TilePick {
   int tile;
   int64_t splits;
+  double us;
 };
-// The tile with the least estimated time; splits > 0 fixes the K chunks,
-// else up to max_splits are tried.
-static Bf3Pick bf3_pick(int64_t M, int64_t N, int64_t K, int64_t batch, int64_t splits, int64_t max_splits, int cus) {
-  Bf3Pick best{kT128, std::max<int64_t>(splits, 1)};
-  double tb = 1e30;
-  for (int tile = 0; tile < kTiles; tile++)
-    for (int64_t sp = std::max<int64_t>(splits, 1); sp <= std::max<int64_t>(splits > 0 ? splits : max_splits, 1); sp++) {
-      const double t = bf3_time(tile, M, N, K, batch, sp, cus);
-      if (t < tb) {
-        tb = t;
-        best = {tile, sp};
-      }
+// The least estimated time of g's shape over the split kernel's tiles (bf3) or
+// the fp32 kernel's, and lo .. hi K chunks.
+static TilePick pick_tile(const GemmArgs& g, bool bf3, int64_t batch, int64_t lo, int64_t hi, int cus) {
+  TilePick best{kT128, lo, 1e30};
+  for (int tile = bf3 ? 0 : kTF32; tile < (bf3 ? kBf3Tiles : kTF32 + 1); tile++)
+    for (int64_t sp = lo; sp <= std::max(lo, hi); sp++) {
+      const double t = tile_time(tile, g.M, g.N, g.K, batch, sp, cus);
+      if (t < best.us) best = {tile, sp, t};
     }
   return best;
 }
+
+// K chunks that a product may be cut into: of at least 256, at most 32 of them.
+static int64_t most_splits(const GemmArgs& g) { return std::max<int64_t>(1, std::min<int64_t>(32, g.K / 256)); }
 
 // Estimated time (us) of gemm_small_kernel: whole rounds of the CUs, each a
 // launch's latency and the wave's share of K (measured: one round of 64 x 32
@@ -1055,9 +1077,7 @@ static double small_time(const GemmArgs& g, int batch, int cus) {
 static bool small_takes(const GemmArgs& g, int batch, int cus) {
   if (g.groups || g.kseg || g.kitems || g.kchunk || g.a_rows || g.c_rows || g.row_scale || g.mask_out || g.K <= 0)
     return false;
-  const int64_t most = std::min<int64_t>(32, g.K / 256);
-  const Bf3Pick p = bf3_pick(g.M, g.N, g.K, batch, 0, g.C2 ? 1 : most, cus);
-  return small_time(g, batch, cus) < 0.8 * bf3_time(p.tile, g.M, g.N, g.K, batch, p.splits, cus);
+  return small_time(g, batch, cus) < 0.8 * pick_tile(g, true, batch, 1, g.C2 ? 1 : most_splits(g), cus).us;
 }
 
 int launch_gemm_ex(const GemmArgs& in, bool tA, bool tB, int batch, hipStream_t s) {
@@ -1071,15 +1091,7 @@ int launch_gemm_ex(const GemmArgs& in, bool tA, bool tB, int batch, hipStream_t 
     set_error("gemm: K blocks must be a multiple of 16 and exclude K-grouped and grouped modes");
     return -1;
   }
-  // float4 staging needs each operand's contiguous extent, leading dimension,
-  // batch stride and base to be 4-float aligned.
-  // (K-grouped segments start anywhere, so a k-contiguous operand needs the
-  // scalar path there.)
-  const bool va = aligned16(g.A) && g.lda % 4 == 0 && g.sA % 4 == 0 && ((tA ? g.M : g.K) % 4 == 0) &&
-                  (tA || !(g.kseg || g.kitems));
-  const bool vb = aligned16(g.B) && g.ldb % 4 == 0 && g.sB % 4 == 0 && ((tB ? g.K : g.N) % 4 == 0) &&
-                  (!tB || !(g.kseg || g.kitems));
-  const bool vec = va && vb && (!g.kblk || (g.sAk % 4 == 0 && g.sBk % 4 == 0));
+  const bool vec = reads_float4(g, tA, tB);
   if (g.kblk && !vec) {
     set_error("gemm: K-blocked operands need 16-byte aligned, 4-float strided operands");
     return -1;
@@ -1100,10 +1112,7 @@ int launch_gemm_ex(const GemmArgs& in, bool tA, bool tB, int batch, hipStream_t 
   }
   const int zs = g.kchunk ? (int)ceil_div(g.K, g.kchunk) : 1;
   const int cus = device_cus();
-  // (each operand's own alignment: a row-contiguous one needs none)
-  const bool ka = tA || (aligned16(g.A) && g.lda % 4 == 0 && g.sA % 4 == 0 && g.K % 4 == 0 && g.sAk % 4 == 0);
-  const bool kb = !tB || (aligned16(g.B) && g.ldb % 4 == 0 && g.sB % 4 == 0 && g.K % 4 == 0 && g.sBk % 4 == 0);
-  if (ka && kb && !(tA && tB) && small_takes(g, batch, cus)) {
+  if (small_reads(g, tA, tB) && small_takes(g, batch, cus)) {
     const int tm = g.M > 32 ? 2 : 1;
     g.tiles_m = (int)ceil_div(g.M, 32 * tm);
     g.tiles_n = (int)ceil_div(g.N, 32);
@@ -1128,7 +1137,7 @@ int launch_gemm_ex(const GemmArgs& in, bool tA, bool tB, int batch, hipStream_t 
   if (bf3 && g.groups) {
     bn = 256;  // 128-row tiles (the caller's tile list), 256 columns
   } else if (bf3 && plain && !g.kitems && !g.kseg) {
-    tile = bf3_pick(g.M, g.N, g.K, batch, zs, zs, cus).tile;
+    tile = pick_tile(g, true, batch, zs, zs, cus).tile;
     bm = tile == kT128 ? 128 : 256;
   }
   g.tiles_m = (int)ceil_div(g.M, bm);
@@ -1194,14 +1203,42 @@ static bool splittable(const GemmArgs& g) {
 // float4 staging aligned).
 static int split_chunk(int K, int splits) { return (int)(ceil_div(ceil_div(K, splits), BK) * BK); }
 
-int gemm_split_count(const GemmArgs& g, int batch) {
-  if (!splittable(g) || g.M <= 0 || g.N <= 0 || batch <= 0) return 1;
-  if (small_takes(g, batch, device_cus())) return 1;
-  // chunks of at least 256, at most 32 of them; the estimate prices the
-  // partial sums against the CUs that a few tiles leave idle
-  const int64_t sp =
-      bf3_pick(g.M, g.N, g.K, batch, 0, std::min<int64_t>(32, g.K / 256), device_cus()).splits;
+// Chunks of at most `sp` that cover K.
+static int chunks_of(const GemmArgs& g, int64_t sp) {
   return sp < 2 ? 1 : (int)ceil_div(g.K, split_chunk(g.K, (int)sp));
+}
+
+// The product of one K chunk: plain, into the workspace.
+static GemmArgs chunk_args(const GemmArgs& in) {
+  GemmArgs p = in;
+  p.mode = kEpiAct;
+  p.act = 0;
+  p.aux = nullptr;
+  p.mask_in = nullptr;  // the reduction applies relu' from aux
+  return p;
+}
+
+// The estimate prices the partial sums against the CUs that a few tiles leave
+// idle, on the kernel that will run the chunks: a count of 1 where
+// gemm_small_kernel takes the product, which needs its operands' alignment (33
+// x 64 x 1201, which it cannot read, on the fp32 kernel: 1 chunk 145 us, 4 54).
+// Over 27 shapes that only the fp32 kernel reads (K 512 to 8192, 1 to 289 tiles)
+// the count's time is within 6% of the best of all counts with chunks of 256.
+int gemm_split_count(const GemmArgs& g, bool tA, bool tB, int batch) {
+  if (!splittable(g) || g.M <= 0 || g.N <= 0 || batch <= 0) return 1;
+  const int cus = device_cus();
+  if (small_reads(g, tA, tB) && small_takes(g, batch, cus)) return 1;
+  const bool bf3 = bf3_takes(chunk_args(g), reads_float4(g, tA, tB), true, tA, tB);
+  return chunks_of(g, pick_tile(g, bf3, batch, 1, most_splits(g), cus).splits);
+}
+
+int gemm_split_most(const GemmArgs& g, int batch) {
+  if (!splittable(g) || g.M <= 0 || g.N <= 0 || batch <= 0) return 1;
+  const int cus = device_cus();
+  int n = 1;
+  for (const bool bf3 : {false, true})
+    n = std::max(n, chunks_of(g, pick_tile(g, bf3, batch, 1, most_splits(g), cus).splits));
+  return n;
 }
 
 size_t gemm_split_workspace(const GemmArgs& g, int batch, int splits) {
@@ -1214,14 +1251,10 @@ int launch_gemm_split(const GemmArgs& in, bool tA, bool tB, int batch, int split
   const int chunk = split_chunk(in.K, splits);
   const int zs = (int)ceil_div(in.K, chunk);
   const int64_t n_out = (int64_t)in.M * in.N;
-  GemmArgs p = in;
+  GemmArgs p = chunk_args(in);
   p.C = ws;
   p.ldc = in.N;
   p.sC = n_out;
-  p.mode = kEpiAct;
-  p.act = 0;
-  p.aux = nullptr;
-  p.mask_in = nullptr;  // the reduction applies relu' from aux
   p.kchunk = chunk;
   p.sCk = n_out * batch;
   if (launch_gemm_ex(p, tA, tB, batch, s) != 0) return -1;

@@ -82,8 +82,10 @@ struct GemmArgs {
 
 int launch_gemm_ex(const GemmArgs& g, bool tA, bool tB, int batch, hipStream_t s);
 // Split-K for GEMMs with few output tiles and a long K: number of K chunks
-// the heuristic picks (1 = no split) and the workspace it needs (floats).
-int gemm_split_count(const GemmArgs& g, int batch);
+// the heuristic picks (1 = no split), the most it picks for the shape whatever
+// the operands' order and alignment, and the workspace of a count (floats).
+int gemm_split_count(const GemmArgs& g, bool tA, bool tB, int batch);
+int gemm_split_most(const GemmArgs& g, int batch);
 size_t gemm_split_workspace(const GemmArgs& g, int batch, int splits);
 // Runs g with `splits` K chunks through `ws` (partials, then a fixed-order
 // reduction applying g's epilogue); splits <= 1 or a plan the split does not

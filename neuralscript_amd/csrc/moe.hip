@@ -934,7 +934,7 @@ static GemmArgs dwg_args(const float* x, const float* dg, float* dWg, int64_t M,
 size_t moe_bwd_splitk_floats(int64_t M, int64_t D, int64_t E) {
   if (M <= 0 || M > INT32_MAX) return 0;
   const GemmArgs g = dwg_args(nullptr, nullptr, nullptr, M, D, E);
-  return gemm_split_workspace(g, 1, gemm_split_count(g, 1));
+  return gemm_split_workspace(g, 1, gemm_split_count(g, true, false, 1));
 }
 
 int launch_moe_backward(const float* x, const float* dout, const float* Wg, const float* We1, const float* We2,
@@ -985,7 +985,7 @@ int launch_moe_backward(const float* x, const float* dout, const float* Wg, cons
   // over K when the caller brought the workspace
   if ((phases & kMoeBwdGate) && dWg) {
     const GemmArgs g = dwg_args(x, b.dg, dWg, M, D, E);
-    const int sp = gemm_split_count(g, 1);
+    const int sp = gemm_split_count(g, true, false, 1);
     const bool split = sp > 1 && b.splitk && gemm_split_workspace(g, 1, sp) <= b.splitk_floats;
     if ((split ? launch_gemm_split(g, true, false, 1, sp, b.splitk, s) : launch_gemm_ex(g, true, false, 1, s)) != 0)
       return -1;

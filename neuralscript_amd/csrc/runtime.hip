@@ -215,7 +215,7 @@ float* scratch(ns_model* m, const std::string& key, size_t n) {
 // GEMMs of the model's plan: split K through a grow-only workspace when the
 // output has too few tiles to fill the device (weight gradients).
 int rt_gemm_ex(ns_model* m, const GemmArgs& g, bool tA, bool tB, int batch) {
-  const int sp = gemm_split_count(g, batch);
+  const int sp = gemm_split_count(g, tA, tB, batch);
   if (sp <= 1) return launch_gemm_ex(g, tA, tB, batch, m->stream);
   float* ws = scratch(m, "splitk", gemm_split_workspace(g, batch, sp));
   if (!ws) return -1;
@@ -1801,15 +1801,10 @@ static GemmArgs plain_gemm(const float* A, const float* B, float* C, int64_t M, 
   return g;
 }
 
-static int split_of(int64_t M, int64_t N, int64_t K, int splits) {
-  if (splits > 0) return splits;
-  return gemm_split_count(plain_gemm(nullptr, nullptr, nullptr, M, N, K, 0, 0, 0, 0), 1);
-}
-
 size_t nsh_op_gemm_splitk_workspace(int64_t M, int64_t N, int64_t K, int splits) {
   if (M <= 0 || N <= 0 || K < 0 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return 0;
-  const int sp = split_of(M, N, K, splits);
-  return gemm_split_workspace(plain_gemm(nullptr, nullptr, nullptr, M, N, K, 0, 0, 0, 0), 1, sp) * sizeof(float);
+  const GemmArgs g = plain_gemm(nullptr, nullptr, nullptr, M, N, K, 0, 0, 0, 0);
+  return gemm_split_workspace(g, 1, splits > 0 ? splits : gemm_split_most(g, 1)) * sizeof(float);
 }
 
 int nsh_op_gemm_splitk(const float* A, const float* B, float* C, int64_t M, int64_t N, int64_t K, int64_t lda,
@@ -1819,12 +1814,12 @@ int nsh_op_gemm_splitk(const float* A, const float* B, float* C, int64_t M, int6
     set_error("gemm_splitk: bad arguments");
     return -1;
   }
-  const int sp = split_of(M, N, K, splits);
+  const GemmArgs g = plain_gemm(A, B, C, M, N, K, lda, ldb, ldc, act);
+  const int sp = splits > 0 ? splits : gemm_split_count(g, transA != 0, transB != 0, 1);
   if (sp > 1 && !workspace) {
     set_error("gemm_splitk: missing workspace");
     return -1;
   }
-  const GemmArgs g = plain_gemm(A, B, C, M, N, K, lda, ldb, ldc, act);
   if (launch_gemm_split(g, transA != 0, transB != 0, 1, sp, (float*)workspace, nullptr) != 0) return -1;
   NSH_CHECK(hipStreamSynchronize(nullptr));
   return 0;

@@ -134,3 +134,31 @@ def test_small_product_of_special_values(variant):
     assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
     calm = np.isfinite(ref) & (np.abs(ref) < 1e30)
     helpers.assert_close(got[calm], ref[calm], f"small gemm beside special values {variant}")
+
+
+# products of few tiles and a long K by the kernel that can read them: the small
+# kernel (aligned; it needs no chunks), and the fp32 kernel, which it must not
+# leave with one chunk (K % 4 != 0, or both transposed)
+@pytest.mark.parametrize("M,N,K,variant,chunks", [(33, 64, 1200, "nn", 1), (33, 64, 1201, "nn", 4),
+                                                  (33, 64, 1201, "nt", 4), (33, 64, 1200, "tt", 4),
+                                                  (33, 64, 1201, "tn", 1), (1501, 160, 1501, "nn", 5),
+                                                  (33, 64, 511, "nn", 1), (33, 64, 512, "tt", 2)])
+def test_chosen_chunks_of_long_products(M, N, K, variant, chunks):
+    """The workspace shows the chunks that were written: `chunks` blocks of M x N
+    floats, inside what nsh_op_gemm_splitk_workspace asked for."""
+    print(f"split count {variant} M={M} N={N} K={K}", flush=True)
+    A, B = operands(M, N, K, 13 * M + K)
+    tA, tB = variant[0] == "t", variant[1] == "t"
+    dA = runtime.DeviceArray.from_host(np.ascontiguousarray(A.T if tA else A))
+    dB = runtime.DeviceArray.from_host(np.ascontiguousarray(B.T if tB else B))
+    dC = runtime.DeviceArray(M * N)
+    need = runtime.lib().nsh_op_gemm_splitk_workspace(M, N, K, 0) // 4
+    ws = runtime.DeviceArray.from_host(np.full(need + 33 * M * N, np.nan, np.float32))
+    runtime.check(runtime.lib().nsh_op_gemm_splitk(dA.ptr, dB.ptr, dC.ptr, M, N, K, M if tA else K, K if tB else N, N,
+                                                   int(tA), int(tB), 0, 0, ws.ptr), "gemm_splitk")
+    written = np.flatnonzero(~np.isnan(ws.to_host()))
+    assert written.size == (chunks * M * N if chunks > 1 else 0)
+    assert written.size == 0 or written[-1] < need
+    a, b = A.astype(np.float64), B.astype(np.float64)
+    bound = (K + 40) * U * (np.abs(a) @ np.abs(b))
+    assert np.all(np.abs(dC.to_host().reshape(M, N).astype(np.float64) - a @ b) <= bound)
