@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <memory>
@@ -82,6 +83,8 @@ struct ns_model {
   std::vector<size_t> last_numel;
   std::vector<Buf> arena;         // per value id
   std::map<std::string, Buf> scratch;
+  // bytes of both, and what they may take together (0: what the device has)
+  size_t buf_bytes = 0, buf_limit = 0;
   std::map<int, int64_t*> dev_idx;  // Index / Scatter index lists on the device, by result id
   nship::HostStage stage;           // pinned staging of the host-pointer entry points' copies
   // Host labels of a host-pointer train call, uploaded when the loss first
@@ -106,13 +109,52 @@ struct ns_model {
 namespace nship {
 namespace {
 
-int ensure(Buf& b, size_t n) {
-  if (n <= b.cap && b.p) return 0;  // (an empty request still gets a buffer)
-  if (b.p) NSH_CHECK(hipFree(b.p));
+size_t buf_size(size_t n) { return (n ? n : 1) * sizeof(float); }  // (an empty request still gets a buffer)
+
+int drop(ns_model* m, Buf& b) {
+  if (!b.p) return 0;
+  NSH_CHECK(hipFree(b.p));  // (waits for the work that uses it)
+  m->buf_bytes -= buf_size(b.cap);
   b.p = nullptr;
   b.cap = 0;
-  NSH_CHECK(hipMalloc(&b.p, (n ? n : 1) * sizeof(float)));
+  return 0;
+}
+
+// b = n floats, b empty before.
+hipError_t take(ns_model* m, Buf& b, size_t n) {
+  hipError_t e = hipErrorOutOfMemory;
+  if (!m->buf_limit || m->buf_bytes + buf_size(n) <= m->buf_limit) e = hipMalloc(&b.p, buf_size(n));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    b.p = nullptr;
+    return e;
+  }
   b.cap = n;
+  m->buf_bytes += buf_size(n);
+  return e;
+}
+
+// Gives back the scratch that a call can do without (optional_scratch).
+int give_back(ns_model* m) {
+  for (const char* key : {"attn_ds", "splitk"}) {
+    auto it = m->scratch.find(key);
+    if (it != m->scratch.end() && drop(m, it->second) != 0) return -1;
+  }
+  return 0;
+}
+
+int ensure(ns_model* m, Buf& b, size_t n) {
+  if (n <= b.cap && b.p) return 0;
+  if (drop(m, b) != 0) return -1;
+  hipError_t e = take(m, b, n);
+  if (e != hipSuccess) {
+    if (give_back(m) != 0) return -1;
+    e = take(m, b, n);
+  }
+  if (e != hipSuccess) {
+    set_error(std::string("hipMalloc: ") + hipGetErrorString(e));
+    return -1;
+  }
   return 0;
 }
 
@@ -208,8 +250,22 @@ struct Frame {
 
 float* scratch(ns_model* m, const std::string& key, size_t n) {
   Buf& b = m->scratch[key];
-  if (ensure(b, n) != 0) return nullptr;
+  if (ensure(m, b, n) != 0) return nullptr;
   return b.p;
+}
+
+// Scratch that the call runs without (more slowly) when there is no room for
+// it: nullptr, and no error.  An eighth more has to be free, for what the call
+// allocates afterwards; the next call looks again.  The pointer is good until
+// the next scratch() or output buffer, which may give it back (ensure).
+float* optional_scratch(ns_model* m, const std::string& key, size_t n) {
+  Buf& b = m->scratch[key];
+  if (n <= b.cap && b.p) return b.p;
+  size_t room = 0, total = 0;
+  if (drop(m, b) != 0 || hipMemGetInfo(&room, &total) != hipSuccess) return nullptr;
+  if (m->buf_limit) room = std::min(room, m->buf_limit - std::min(m->buf_limit, m->buf_bytes));
+  if (room - room / 9 < buf_size(n)) return nullptr;
+  return take(m, b, n) == hipSuccess ? b.p : nullptr;
 }
 
 // GEMMs of the model's plan: split K through a grow-only workspace when the
@@ -217,8 +273,8 @@ float* scratch(ns_model* m, const std::string& key, size_t n) {
 int rt_gemm_ex(ns_model* m, const GemmArgs& g, bool tA, bool tB, int batch) {
   const int sp = gemm_split_count(g, tA, tB, batch);
   if (sp <= 1) return launch_gemm_ex(g, tA, tB, batch, m->stream);
-  float* ws = scratch(m, "splitk", gemm_split_workspace(g, batch, sp));
-  if (!ws) return -1;
+  // (without the workspace it runs unsplit)
+  float* ws = optional_scratch(m, "splitk", gemm_split_workspace(g, batch, sp));
   return launch_gemm_split(g, tA, tB, batch, sp, ws, m->stream);
 }
 
@@ -283,7 +339,7 @@ float* out_buf(ns_model* m, Frame& fr, int id, size_t n) {
     fr.ptr[id] = fr.direct;
     return fr.direct;
   }
-  if (ensure(m->arena[id], n) != 0) return nullptr;
+  if (ensure(m, m->arena[id], n) != 0) return nullptr;
   fr.numel[id] = n;
   fr.ptr[id] = m->arena[id].p;
   return fr.ptr[id];
@@ -670,14 +726,13 @@ int attention_backward(ns_model* m, Frame& fr, const Instr& I, AttnGrads* out) {
   }
   {
     Prof p(m, "attention_bwd");
-    const size_t nds = attention_bwd_ds_floats(BS, D, H);
-    // no room for dS: the pass that recomputes S and dP for dQ
-    float* ds = nds ? scratch(m, "attn_ds", nds) : nullptr;
-    if (nds && !ds) (void)hipGetLastError();
     const void* rd[5] = {sv.qkv, sv.qkv + BS * D, sv.qkv + 2 * BS * D, sv.ctx, dPre};
     float* pad = nullptr;
     if (!attention_in_place(D, H, D, rd, 5) && !(pad = scratch(m, "attn_pad", attention_pad_floats(BS, D, H, true))))
       return -1;
+    // no room for dS: the pass that recomputes S and dP for dQ
+    const size_t nds = attention_bwd_ds_floats(BS, D, H);
+    float* ds = nds ? optional_scratch(m, "attn_ds", nds) : nullptr;
     if (launch_attention_bwd(sv.qkv, sv.qkv + BS * D, sv.qkv + 2 * BS * D, sv.ctx, dPre, sv.lse, delta, dqkv,
                              dqkv + BS * D, dqkv + 2 * BS * D, BS, D, H, D, ds, pad, s) != 0)
       return -1;
@@ -775,9 +830,14 @@ int optimizer_step(ns_model* m, Frame& fr, const Instr& I, float lr) {
       max_elems = std::max(max_elems, n);
     } else {
       auto& st = m->adam[wid];
-      if (!st.m) {
-        NSH_CHECK(hipMalloc(&st.m, (size_t)n * sizeof(float)));
-        NSH_CHECK(hipMalloc(&st.v, (size_t)n * sizeof(float)));
+      if (!st.v) {  // (a step that ran out of room in between has m alone)
+        for (float** p : {&st.m, &st.v}) {
+          if (*p || hipMalloc(p, (size_t)n * sizeof(float)) == hipSuccess) continue;
+          (void)hipGetLastError();
+          *p = nullptr;
+          if (give_back(m) != 0) return -1;
+          NSH_CHECK(hipMalloc(p, (size_t)n * sizeof(float)));
+        }
         NSH_CHECK(hipMemsetAsync(st.m, 0, (size_t)n * sizeof(float), s));
         NSH_CHECK(hipMemsetAsync(st.v, 0, (size_t)n * sizeof(float), s));
       }
@@ -1290,6 +1350,8 @@ ns_model* nsh_model_init(const nsh_plan* ph, const float* weights, size_t num_fl
     return nullptr;
   }
   ns_model* m = new ns_model();
+  // (so that small cases can run out of room)
+  if (const char* e = std::getenv("NSHIP_MODEL_BUFFER_BYTES")) m->buf_limit = (size_t)std::max(0ll, std::atoll(e));
   m->plan = &P;
   m->arena.resize(P.vals.size());
   bool ok = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) == hipSuccess;
@@ -1366,7 +1428,7 @@ int nsh_eval_infer(ns_model* m, const float* input, float* output, size_t input_
     return -1;
   }
   Buf& xb = m->scratch["__x"];
-  if (ensure(xb, input_numel) != 0) return -1;
+  if (ensure(m, xb, input_numel) != 0) return -1;
   if (stage_h2d(m->stage, xb.p, input, input_numel * sizeof(float), m->stream) != 0) return -1;
   float* res = nullptr;
   size_t n = 0;
@@ -1552,7 +1614,7 @@ static int stage_train_inputs(ns_model* m, const float* input, const float* labe
   const size_t ny = rows * (size_t)P.out_cols;
   Buf& xb = m->scratch["__x"];
   Buf& yb = m->scratch["__y"];
-  if (ensure(xb, input_numel) != 0 || ensure(yb, ny) != 0) return -1;
+  if (ensure(m, xb, input_numel) != 0 || ensure(m, yb, ny) != 0) return -1;
   if (!m->before_ev) NSH_CHECK(hipEventCreateWithFlags(&m->before_ev, hipEventDisableTiming));
   NSH_CHECK(hipEventRecord(m->before_ev, m->stream));
   if (stage_h2d(m->stage, xb.p, input, input_numel * sizeof(float), m->stream) != 0) return -1;
