@@ -1004,10 +1004,18 @@ static int device_cus() {
 // general epilogue's activations stay on the fp32 kernel, and so do products
 // that ask for it (GemmArgs::f32).
 // Short K: one MFMA aligns its 16 products to the largest and drops what lies
-// below fp32's last place there.  Over a long sum that is far below the
-// roundings of the sum itself; a short sum with one dominant term is left
-// with about 1.4 x 2^-24 instead of 0.5 (K = 16, lognormal operands: relative
-// error 8.5e-8), and its product is bound by its memory traffic either way.
+// below fp32's last place there, and the split drops up to 2^-24 of a product
+// (split3.h).  Over a long sum both are far below the roundings of the sum
+// itself; a short one with a dominant term has up to 1.8 x 2^-24 instead of
+// 1.0, and its product is bound by its memory traffic either way.
+// Long sums against float64, 2-norm in units of 2^-24, fp32 MFMA -> this, 2048 x
+// 2048 outputs: N(0, 1), K = 128 3.4 -> 1.1, 512 6.8 -> 2.1, 4096 9.6 -> 4.6; e^(2
+// N(0, 1)), 512 12.5 -> 2.7, 4096 32 -> 4.3; softmax(N(0, 1)) less one-hot, 4096 9.7
+// -> 5.0; the gradients of an output layer of 8192 classes 5.9..9.6 -> 3.3..5.3.
+// Few large terms among thousands that vanish beside them are the exception:
+// softmax(8 N(0, 1)) less one-hot, 512 2.9 -> 2.2, but 2048 2.3 -> 2.6 and 4096 2.7
+// -> 3.2 (a slab's leading products summed apart and added by VALU: 2.3 and 2.8,
+// every product 7 to 10% slower).
 constexpr int kBf3MinK = 128;
 static bool bf3_takes(const GemmArgs& g, bool vec, bool plain, bool tA, bool tB) {
   if (!vec || (tA && tB) || g.f32 || g.K < kBf3MinK) return false;

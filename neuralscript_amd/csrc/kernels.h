@@ -74,8 +74,7 @@ struct GemmArgs {
   // separately stored products, e.g. dX = [dQ dK dV] . [Wq Wk Wv]^T.
   int kblk = 0;
   int64_t sAk = 0, sBk = 0;
-  // fp32 MFMA only: operands whose sums a few terms dominate (a top-1
-  // router's gradient), where three bf16 pieces cost a bit of the last place
+  // fp32 MFMA only (a top-1 router's gradients: moe.hip)
   bool f32 = false;
   int tiles_m = 0, tiles_n = 0;    // filled by the launcher
 };

@@ -1,13 +1,18 @@
 // fp32 products on the bf16 matrix cores: every fp32 operand is written as
 // the sum of three bf16 pieces (8 significand bits each, 24 together), and a
-// product a b is accumulated in fp32 from six of the nine piece products.
+// product a b is accumulated in fp32 from six of the nine piece products (the
+// method of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial
+// intelligence datatype for higher-precision computations", ARITH 2019).
 //
 //   a = a0 + a1 + a2,  a0 = bf16(a), a1 = bf16(a - a0), a2 = a - a0 - a1
 //   a b ~ a0 b2 + a2 b0 + a1 b1 + a0 b1 + a1 b0 + a0 b0
 //
-// The pieces are round-to-nearest, so |a1| <= 2^-9 |a| and |a2| <= 2^-18 |a|:
+// The pieces are round-to-nearest, so |a1| <= 2^-8 |a| and |a2| <= 2^-17 |a|:
 // the split is exact (no operand bit is dropped) and the three products left
-// out are at most 2^-26 |a b| together, a quarter of one fp32 rounding.
+// out are at most 2^-24 |a b| together, one fp32 rounding (0.99 of it at a = b =
+// 0x1.00ff8p+0); their root mean square over the significands is 2^-27.5 |a b|.
+// So a product that stands alone has a largest error of 2 x 2^-24, measured
+// 1.77 (fp32 MFMA 1.00), and the same root mean square, 0.42.
 // gfx950's 32x32x16 bf16 MFMA runs 16 times the rate of the 32x32x2 fp32 one,
 // so six of them take 6/16 of the time, and it rounds its accumulator once
 // per 16 products where the fp32 one rounds once per 2.  Measured against

@@ -9,6 +9,7 @@ largest value covers the roundings, where the tests above this file's allow
 import numpy as np
 import pytest
 
+import split3_model as sm
 from neuralscript_amd import runtime, synth
 from neuralscript_amd.runtime import DeviceArray as DA
 
@@ -148,6 +149,19 @@ def test_gradient_tile_edges(S, dk, store_ds):
     H = 2
     arrs = inputs(S, H * dk, 17 * S + dk, 4)
     assert_gradients(arrs, H, gradients(*arrs, H, store_ds))
+
+
+@pytest.mark.parametrize("S", [64, 130, 500])
+@pytest.mark.parametrize("dk", [32, 64, 128])
+@pytest.mark.parametrize("store_ds", [0, 1])
+def test_every_piece_counts(S, dk, store_ds):
+    """The bounds that a lost product of pieces breaks (test_split_bounds.py)."""
+    print(f"precise attention S={S} dk={dk} store_ds={store_ds}", flush=True)
+    arrs = inputs(S, dk, 7 * S + dk, 4)
+    refs = sm.attention(*arrs)
+    assert sm.rel(core(*arrs[:3], 1)[0], refs[0]) <= sm.FORWARD_BOUND
+    for name, g, r in zip(("dQ", "dK", "dV"), gradients(*arrs, 1, store_ds), refs[1:]):
+        assert sm.rel(g, r) <= sm.BACKWARD_BOUND, name
 
 
 @pytest.mark.parametrize("dk", [32, 64])

@@ -3,13 +3,16 @@ float64, and on the values its pieces cannot hold, against the oracle.
 
 Bound of a result: every fp32 rounding of the accumulator is at most 2^-24 of
 the running sum of |a b|, six piece products per 16 of k and one more for each
-K chunk; the three dropped piece products are at most 2^-26 |a b|.
+K chunk; the three dropped piece products are at most 2^-24 |a b| together.
+That finds a wrong element, not a lost piece, whose size is 2^-17 |a b|: the
+bounds of split3_model do.
 """
 import numpy as np
 import pytest
 
 import helpers
 import oracle
+import split3_model as sm
 from neuralscript_amd import runtime, synth
 
 pytestmark = pytest.mark.gpu
@@ -53,6 +56,33 @@ def test_split_product_against_float64(M, N, K, variant):
     a, b = A[rows].astype(np.float64), B.astype(np.float64)
     bound = (6 * (K // 16 + 1) + 4) * U * (np.abs(a) @ np.abs(b))
     assert np.all(np.abs(got - a @ b) <= bound)
+
+
+# on the small kernel, on 256- and 128-row tiles, over K chunks
+PRECISE = [(256, 512, 128, None), (40, 72, 2048, None), (2048, 2048, 256, None), (4096, 1028, 132, None),
+           (1500, 516, 512, None), (1024, 1028, 4096, 0), (260, 132, 1032, 4)]
+
+
+@pytest.mark.parametrize("M,N,K,splits", PRECISE)
+@pytest.mark.parametrize("variant", ["nn", "nt", "tn"])
+def test_every_piece_counts_on_normal_operands(M, N, K, splits, variant):
+    print(f"precise gemm {variant} M={M} N={N} K={K}", flush=True)
+    A, B = operands(M, N, K, 3 * M + N + K)
+    got = product(A, B, variant, splits)
+    assert sm.rel(got, A.astype(np.float64) @ B.astype(np.float64)) <= sm.normal_bound(K)
+
+
+@pytest.mark.parametrize("M,N,K,splits", PRECISE)
+@pytest.mark.parametrize("variant", ["nn", "nt", "tn"])
+def test_every_piece_counts_in_products_of_one_term(M, N, K, splits, variant):
+    """Row m of A holds one value, at k = m mod K, of 24 significant bits."""
+    rng = np.random.default_rng(M + K)
+    B = (1 + rng.random((K, N))).astype(np.float32) * rng.choice(np.float32([-1, 1]), (K, N))
+    A, k, a = np.zeros((M, K), np.float32), np.arange(M) % K, (1 + rng.random(M)).astype(np.float32)
+    a[0] = B[0, 0] = float.fromhex("0x1.00ff8p+0")  # where the dropped products weigh most
+    A[np.arange(M), k] = a
+    ref = a[:, None].astype(np.float64) * B[k]
+    assert np.max(np.abs(product(A, B, variant, splits) / ref - 1)) <= sm.one_term_bound()
 
 
 @pytest.mark.parametrize("M,N,K,splits", [(128, 128, 512, 3), (260, 132, 1032, 4), (512, 512, 4096, 0)])
