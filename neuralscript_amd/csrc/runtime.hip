@@ -1877,10 +1877,14 @@ int nsh_op_gemm_splitk(const float* A, const float* B, float* C, int64_t M, int6
     return -1;
   }
   const GemmArgs g = plain_gemm(A, B, C, M, N, K, lda, ldb, ldc, act);
-  const int sp = splits > 0 ? splits : gemm_split_count(g, transA != 0, transB != 0, 1);
+  int sp = splits > 0 ? splits : gemm_split_count(g, transA != 0, transB != 0, 1);
   if (sp > 1 && !workspace) {
-    set_error("gemm_splitk: missing workspace");
-    return -1;
+    // (chunks that only the operands' alignment asks for are not insisted on)
+    if (splits > 0 || gemm_split_count(plain_gemm(nullptr, nullptr, nullptr, M, N, K, 0, 0, 0, 0), true, false, 1) > 1) {
+      set_error("gemm_splitk: missing workspace");
+      return -1;
+    }
+    sp = 1;
   }
   if (launch_gemm_split(g, transA != 0, transB != 0, 1, sp, (float*)workspace, nullptr) != 0) return -1;
   NSH_CHECK(hipStreamSynchronize(nullptr));

@@ -192,3 +192,16 @@ def test_chosen_chunks_of_long_products(M, N, K, variant, chunks):
     a, b = A.astype(np.float64), B.astype(np.float64)
     bound = (K + 40) * U * (np.abs(a) @ np.abs(b))
     assert np.all(np.abs(dC.to_host().reshape(M, N).astype(np.float64) - a @ b) <= bound)
+
+
+def test_split_without_a_workspace():
+    """Refused where the shape asks for chunks, run unsplit where only the
+    operands' alignment does."""
+    for M, N, K, refused in [(33, 64, 1201, False), (512, 512, 4096, True)]:
+        A, B = operands(M, N, K, K)
+        dA, dB, dC = runtime.DeviceArray.from_host(A), runtime.DeviceArray.from_host(B), runtime.DeviceArray(M * N)
+        rc = runtime.lib().nsh_op_gemm_splitk(dA.ptr, dB.ptr, dC.ptr, M, N, K, K, N, N, 0, 0, 0, 0, None)
+        assert (rc != 0) == refused
+        if not refused:
+            a, b = A.astype(np.float64), B.astype(np.float64)
+            assert np.all(np.abs(dC.to_host().reshape(M, N) - a @ b) <= (K + 8) * U * (np.abs(a) @ np.abs(b)))
