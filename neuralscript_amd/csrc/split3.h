@@ -16,10 +16,10 @@
 // gfx950's 32x32x16 bf16 MFMA runs 16 times the rate of the 32x32x2 fp32 one,
 // so six of them take 6/16 of the time, and it rounds its accumulator once
 // per 16 products where the fp32 one rounds once per 2.  Measured against
-// float64 on one 32x32 tile of N(0,1) operands (relative 2-norm error, fp32
-// MFMA -> this): K = 16 7.4e-8 -> 3.4e-8, 64 1.5e-7 -> 1.1e-7, 512 4.1e-7 ->
-// 3.4e-7, 4096 1.2e-6 -> 1.0e-6, 16384 2.3e-6 -> 2.1e-6; uniform [0, 1)
-// operands 6.2e-8 -> 3.2e-8, ..., 1.7e-6 -> 1.1e-6.
+// float64 on one 32x32 tile of N(0,1) operands with one accumulator (relative
+// 2-norm error, fp32 MFMA -> this): K = 16 7.4e-8 -> 3.4e-8, 64 1.5e-7 ->
+// 1.1e-7, 512 4.1e-7 -> 3.4e-7, 4096 1.2e-6 -> 1.0e-6, 16384 2.3e-6 -> 2.1e-6;
+// uniform [0, 1) operands 6.2e-8 -> 3.2e-8, ..., 1.7e-6 -> 1.1e-6.
 //
 // Operands are scaled by kSplitUp = 2^24 before they are split, and the sums by
 // kSplitDown = 2^-48 (all exact): the last piece then stays above bf16's
